@@ -140,3 +140,26 @@ def test_audio_round_trip_matches_oracle(native, oracle, stereo):
     assert len(fast) == 8 + (frames * 12 * 10 + 7) // 8
     fast_pcm, _ = dac.decode(session, fast)
     assert np.array_equal(_bits(fast_pcm), _bits(pcm))
+
+
+@pytest.mark.parametrize("synthesis", [False, True])
+@pytest.mark.parametrize("frames", [33, 130, 450, 1400])
+def test_convolution_tiles_agree_across_sizes(stereo, mono, synthesis, frames):
+    """The convolutions choose their tile by the grid it makes, so windows of
+    different lengths take different tiles (and leave different remainders): the
+    frames a short window shares with a long one, past the reference's context
+    frames, are the same bits. The short windows' sizes are held against the oracle
+    above."""
+    for parts in (stereo, mono):
+        _, _, session, dac, _, _ = parts
+        rng = np.random.default_rng(frames)
+        if synthesis:
+            signal, step, left, right = rng.standard_normal((frames, 1024)).astype(np.float32), 1, 11, 11
+        else:
+            signal, step, left, right = _pcm(frames * 512 / 44100, dac.channels, 9, frames), 512, 8, 9
+        long = dac.apply(session, synthesis, signal, frames * step).reshape(frames, -1)
+        for begin, count in ((0, 2), (frames // 2, 5), (frames - 1, 1)):
+            low, high = max(0, begin - left), min(frames, begin + count + right)
+            window = np.ascontiguousarray(signal[low * step:high * step])
+            short = dac.apply(session, synthesis, window, (high - low) * step).reshape(high - low, -1)
+            assert np.array_equal(_bits(short[begin - low:begin - low + count]), _bits(long[begin:begin + count]))

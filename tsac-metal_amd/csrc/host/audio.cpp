@@ -198,7 +198,7 @@ DacModel::DacModel(unsigned channels, unsigned books, const DacConvolutionSource
     require(books >= 1 && books <= (channels == 1 ? 9u : 12u), "DAC model codebooks out of range");
     require(analysis && synthesis && analysis_alpha && synthesis_alpha && rvq, "missing DAC model tensor");
     check_hip(hipGetDevice(&device_), "hipGetDevice");
-    // Layout: every convolution's w[tap][in][out_padded] and bias, then every
+    // Layout: every convolution's w[tap][in][columns] and bias, then every
     // activation's alpha, each 256-byte aligned.
     const auto align = [](std::size_t n) { return (n + 255) / 256 * 256; };
     std::size_t bytes = 0;
@@ -208,9 +208,8 @@ DacModel::DacModel(unsigned channels, unsigned books, const DacConvolutionSource
         for (unsigned i = 0; i < 30; ++i)
         {
             const ConvShape s = dac_conv_shape(g == 1, channels, i);
-            const std::size_t padded = (s.out + dac_channel_block - 1) / dac_channel_block * dac_channel_block;
             offsets.push_back(bytes);
-            bytes += align(std::size_t(s.kernel) * s.in * padded * 4) + align(std::size_t(s.out) * 4);
+            bytes += align(dac_conv_elements(s) * 4) + align(std::size_t(s.out) * 4);
         }
     }
     for (unsigned g = 0; g < 2; ++g)
@@ -230,19 +229,19 @@ DacModel::DacModel(unsigned channels, unsigned books, const DacConvolutionSource
         for (unsigned i = 0; i < 30; ++i)
         {
             const ConvShape s = dac_conv_shape(g == 1, channels, i);
-            const int padded = (s.out + dac_channel_block - 1) / dac_channel_block * dac_channel_block;
+            const int columns = dac_conv_columns(s);
             const std::vector<float> prepared = prepare_dac_convolution(sources[i], s);
             for (int o = 0; o < s.out; ++o)
             {
                 require(std::isfinite(sources[i].bias[o]), "nonfinite DSP value");
             }
-            layout.assign(std::size_t(s.kernel) * s.in * padded, 0.0f);
-            dac_conv_layout(s, prepared.data(), layout.data(), padded);
+            layout.resize(dac_conv_elements(s));
+            dac_conv_layout(s, prepared.data(), layout.data(), columns);
             uint8_t* w = base + offsets[g * 30 + i];
             uint8_t* b = w + align(layout.size() * 4);
             check_hip(hipMemcpy(w, layout.data(), layout.size() * 4, hipMemcpyHostToDevice), "upload DAC weights");
             check_hip(hipMemcpy(b, sources[i].bias, std::size_t(s.out) * 4, hipMemcpyHostToDevice), "upload DAC bias");
-            convolutions_.push_back({s, reinterpret_cast<const float*>(w), reinterpret_cast<const float*>(b), padded});
+            convolutions_.push_back({s, reinterpret_cast<const float*>(w), reinterpret_cast<const float*>(b), columns});
         }
     }
     constexpr float epsilon = std::bit_cast<float>(uint32_t{0x3089705f});

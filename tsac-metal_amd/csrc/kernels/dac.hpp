@@ -18,7 +18,7 @@
 
 namespace tsac_hip
 {
-// Output channels one wave computes (weights padded to a multiple).
+// The columns of a convolution's weights are padded to a multiple.
 constexpr int dac_channel_block = 16;
 
 struct ConvShape
@@ -39,14 +39,28 @@ struct ConvShape
     }
 };
 
-// Device weights of one convolution: w[tap][in][out_padded] (out fastest,
-// out_padded a multiple of dac_channel_block, zero beyond `out`), bias [out].
+// Columns of a convolution's device weights: an ordinary one's output channels,
+// a transposed one's (channel, residue of the stride) pairs, padded.
+inline int dac_conv_columns(const ConvShape& s)
+{
+    const int columns = s.transposed ? s.out * s.stride : s.out;
+    return (columns + dac_channel_block - 1) / dac_channel_block * dac_channel_block;
+}
+
+// Floats of its device weights.
+inline std::size_t dac_conv_elements(const ConvShape& s)
+{
+    return std::size_t(s.transposed ? s.kernel / s.stride : s.kernel) * s.in * dac_conv_columns(s);
+}
+
+// Device weights of one convolution: w[tap][in][columns] (columns fastest, zero
+// beyond the last one), tap the ordinary tap or, transposed, tap / stride; bias [out].
 struct ConvWeights
 {
     ConvShape shape;
     const float* w = nullptr;
     const float* bias = nullptr;
-    int out_padded = 0;
+    int columns = 0;
 };
 
 struct Strided
@@ -80,8 +94,8 @@ struct ConvArgs
 void dac_conv(const ConvArgs& args, hipStream_t stream);
 
 // Host re-layout of a prepared convolution (stored axes, axis 0 fastest:
-// ordinary [in, kernel, out], transposed [out, kernel, in]) into w[tap][in][out_padded].
-void dac_conv_layout(const ConvShape& shape, const float* stored, float* device_layout, int out_padded);
+// ordinary [in, kernel, out], transposed [out, kernel, in]) into w[tap][in][columns].
+void dac_conv_layout(const ConvShape& shape, const float* stored, float* device_layout, int columns);
 
 // RVQ tensors of one codebook on the device.
 struct RvqBook
