@@ -240,7 +240,7 @@ int tsac_hip_prepare_rvq(const float* codebook, const float* in_v, const float* 
 
 /* analyze_audio (src/common/audio_pipeline.hpp:37-58) on the GPU: padded PCM,
  * interleaved float [frames*512][groups*dac channels], through DAC analysis and
- * the quantizer in chunks of 400 latent frames with 8/9 context frames, to
+ * the quantizer in chunks of latent frames with 8/9 context frames, to
  * tokens [frame][group][codebook] (frames*groups*codebooks). */
 int tsac_hip_dac_analyze(tsac_hip_session* session, const tsac_hip_dac* dac, const float* pcm, size_t frames,
                          size_t groups, uint32_t codebooks, uint16_t* tokens);
