@@ -546,3 +546,41 @@ def test_calibration_probes(torch, native):
     torch.cuda.synchronize()
     with pytest.raises(native.HipError, match="multiple of 64 KiB"):
         native.probe_read(data[:1000])
+
+
+@pytest.mark.parametrize("heads,hw", [(16, 64), (4, 128)])
+@pytest.mark.parametrize("lengths,kind", [([65, 31, 33, 64, 1] * 8, "normal"), ([330], "normal"), ([129, 96], "spread"),
+                                          ([100], "dead infinity"), ([70], "zeros"), ([65], "tiny")])
+def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, kind):
+    """The causal kernel's own choices: 4 or 8 waves by the grid, edges of its 32-query
+    and 64-key tiles, scores more than 87 below the maximum (where weights and their
+    sums meet subnormals), and the last block's dead keys, whose values may be
+    infinite, and whose terms must not turn a zero sum's sign."""
+    rng = np.random.default_rng(sum(lengths) + hw)
+    w, rows = heads * hw, sum(lengths)
+    qkv = rng.standard_normal((rows, 3 * w)).astype(np.float32)
+    if kind == "spread":
+        qkv[:, :w] *= 60
+    elif kind == "dead infinity":
+        qkv[90, 2 * w:] = np.inf
+    elif kind == "zeros":
+        qkv[:, 2 * w:2 * w + hw] = 0
+        qkv[::3, 2 * w + hw:] *= -0.0
+    elif kind == "tiny":
+        qkv[:, :w] *= 60
+        qkv[:, 2 * w:] *= 1e-38
+    qkv = bf16_bits(qkv)
+    starts = np.cumsum([0] + lengths[:-1]).astype(np.int32)
+    scale = np.float32(1 / np.sqrt(hw))
+    out = empty(torch, (rows, w), torch.int16)
+    native.attention_causal(dev(torch, qkv), heads, hw, dev(torch, starts), dev(torch, np.array(lengths, np.int32)),
+                            dev(torch, np.zeros(len(lengths), np.int32)), len(lengths), max(lengths), None, scale, out)
+    got = host(out)
+    for start, length in list(zip(starts, lengths))[:5]:
+        seq = qkv[start:start + length]
+        q, k, v = seq[:, :w].copy(), seq[:, w:2 * w].copy(), seq[:, 2 * w:].copy()
+        for t in range(length):
+            expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, False)
+            finite = np.isfinite(bf16_float(expected))
+            assert np.array_equal(got[start + t][finite], expected[finite]), (length, t)
+            assert not np.isfinite(bf16_float(got[start + t][~finite])).any()

@@ -10,8 +10,8 @@
 // Decode (one query per sequence): each (sequence, head)'s 64-key blocks are
 // spread over several workgroups of one launch, one wave per block; the last
 // workgroup to arrive merges the block records in ascending order.
-// Prefill (encode, all queries known): one workgroup per (sequence, head,
-// 64-query tile) walks the causal key blocks with Q/K/V tiles in LDS.
+// Prefill (encode, all queries known): one workgroup per (sequence, head, 32-query
+// tile), one wave per causal key block, the blocks' sums merged in ascending order.
 #include "attention.hpp"
 #include "device_numeric.hpp"
 
@@ -64,6 +64,7 @@ __global__ void append_kernel(const uint16_t* __restrict__ qkv, int rows, int wi
 }
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Waves per decode workgroup; each wave computes one 64-key block's record.
 constexpr int decode_waves = 4;
@@ -421,354 +422,515 @@ __global__ __launch_bounds__(decode_waves * 64) void decode_attention_kernel(
 
 // ------------------------------------------------------------------ prefill
 
-constexpr int tile = 64;
+constexpr int tile = 64;                          // keys of a block
+constexpr int per_lane = 4, queries = 8 * per_lane; // of a wave
 
-// With 64-wide heads the key tile is widened to fp32 as it is stored, once
-// per block, instead of by each of the 16 threads that read a key row (the
-// workgroup still fits three to a CU); 128-wide heads keep BF16 keys.
-template <int HW> constexpr bool wide_keys = HW == 64;
-
-template <int HW> struct PrefillShared
+// 16 bytes at any 2-byte-aligned address.
+__device__ __forceinline__ u32x4 load16(const uint16_t* from)
 {
-    static constexpr int row = HW + 8;  // BF16 elements per LDS row (16-byte pad)
-    static constexpr int key_row = HW + 4; // fp32 elements per widened key row
-    uint16_t q[tile * row];
-    uint16_t k[wide_keys<HW> ? 8 : tile * row];
-    float kf[wide_keys<HW> ? tile * key_row : 4];
-    uint16_t v[tile * row];
-    float p[tile][tile + 4];
-};
+    u32x4 u;
+    __builtin_memcpy(&u, from, 16);
+    return u;
+}
 
-// Loads a [64][HW] tile from rows of `source` (row stride `stride` elements)
-// with optional rotary at positions first..first+63. Rows at or beyond `limit`
-// are zero. With a float destination the values are stored widened (rows of
-// key_row floats).
-template <int HW, class T>
-__device__ __forceinline__ void load_tile(T* dst, const uint16_t* source, std::size_t stride,
-                                          int first, int limit, const uint16_t* rotations)
+// Rotary (optional) of eight consecutive values.
+__device__ __forceinline__ u32x4 rotate8(u32x4 u, u32x4 coefficients)
 {
-    constexpr bool widen = sizeof(T) == 4;
-    constexpr int row = widen ? PrefillShared<HW>::key_row : PrefillShared<HW>::row;
-    constexpr int chunks = HW / 8;
-    for (int i = threadIdx.x; i < tile * chunks; i += blockDim.x)
-    {
-        const int r = i / chunks, c = i % chunks;
-        const int position = first + r;
-        uint4 u = make_uint4(0, 0, 0, 0);
-        if (position < limit)
-        {
-            u = *reinterpret_cast<const uint4*>(source + std::size_t(position) * stride + c * 8);
-            if (rotations)
-            {
-                uint32_t w[4] = {u.x, u.y, u.z, u.w};
-                const uint16_t* coefficients = rotations + std::size_t(position) * HW + c * 8;
 #pragma unroll
-                for (int p = 0; p < 4; ++p)
-                {
-                    float re = bf16_to_float(uint16_t(w[p] & 0xffff));
-                    float im = bf16_to_float(uint16_t(w[p] >> 16));
-                    rotate_pair(re, im, coefficients + 2 * p);
-                    w[p] = float_to_bf16(re) | (uint32_t(float_to_bf16(im)) << 16);
-                }
-                u = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-        }
-        if constexpr (widen)
-        {
-            const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-            float4* out = reinterpret_cast<float4*>(dst + r * row + c * 8);
-            out[0] = make_float4(__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u),
-                                 __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u));
-            out[1] = make_float4(__uint_as_float(w[2] << 16), __uint_as_float(w[2] & 0xffff0000u),
-                                 __uint_as_float(w[3] << 16), __uint_as_float(w[3] & 0xffff0000u));
-        }
-        else
-        {
-            *reinterpret_cast<uint4*>(dst + r * row + c * 8) = u;
-        }
+    for (int p = 0; p < 4; ++p)
+    {
+        float re = bf16_to_float(uint16_t(u[p] & 0xffff));
+        float im = bf16_to_float(uint16_t(u[p] >> 16));
+        const uint16_t pair[2] = {uint16_t(coefficients[p] & 0xffff), uint16_t(coefficients[p] >> 16)};
+        rotate_pair(re, im, pair);
+        u[p] = float_to_bf16(re) | (uint32_t(float_to_bf16(im)) << 16);
+    }
+    return u;
+}
+
+__device__ __forceinline__ void widen8(u32x4 u, float (&v)[8])
+{
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+    {
+        v[2 * p] = __uint_as_float(u[p] << 16);
+        v[2 * p + 1] = __uint_as_float(u[p] & 0xffff0000u);
     }
 }
 
-// Workgroup of 256 threads: thread t owns queries 4*(t/16)..+3 and, for scores,
-// keys (t%16) + 16*b (b = 0..3) of the current block; for value sums it owns
-// coordinates (t%16)*HW/16 .. +HW/16 of the same four queries. With that key
-// placement the 16-lane butterfly on each register followed by the register
-// pair tree is exactly the balanced pair tree over the block's 64 positions.
-template <int HW>
-__global__ __launch_bounds__(256) void prefill_kernel(
+// One wave's LDS accesses are served in order; this keeps the compiler from
+// moving them across a change of a wave's own tile.
+__device__ __forceinline__ void tile_fence()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// LDS of a workgroup of W waves: the query tile, each wave's key (32
+// coordinates of 64 keys at a time), weight (16 keys x 32 queries, in the keys'
+// place) and value tiles (16 keys x 64 coordinates), and the merged state that
+// the waves hand on block by block. Rows are padded so that eight lanes reading or
+// writing 16 bytes of eight rows meet eight different 16-byte banks.
+constexpr int phase_coordinates = 32, chunk_keys = 16, value_coordinates = 64;
+
+template <int HW, int W> struct PrefillShared
+{
+    static constexpr int q_row = HW + 8, k_row = phase_coordinates + 8, p_row = queries + 4;
+    union Wave
+    {
+        uint16_t k[tile * k_row];
+        struct
+        {
+            float p[chunk_keys * p_row];
+            uint16_t v[chunk_keys * value_coordinates];
+        };
+    };
+    alignas(16) uint16_t q[queries * q_row];
+    alignas(16) Wave wave[W];
+    alignas(16) f32x4 numerator[HW / 64 * per_lane * 2][64]; // per lane: the lane's own sums
+    float maximum[queries], total[queries];
+    int turn[HW / value_coordinates];
+};
+
+// A workgroup takes 32 queries of one (sequence, head); its W waves take the
+// causal 64-key blocks in turn, each whole: lane (lq, lk) = (lane / 8, lane % 8)
+// holds queries lq + 8 a and, for scores, keys lk + 8 b, so that the 8-lane
+// butterfly on each register followed by the register pair tree is exactly the
+// balanced pair tree over the block's 64 positions; for value sums it holds eight
+// coordinates of the same queries. The block's sums join the running state in
+// ascending block order: a wave waits for its block's turn, which the wave of the
+// block before passes on, so the first block's wave never waits and every wait ends.
+//
+// Bound by VALU issue: 59-70 T fma/s on register operands for the whole chip (the
+// chains over coordinates and keys leave no room for matrix instructions), one
+// instruction per 4.3 cycles from one wave, which makes a block 60 k cycles and the
+// longest query tile's rounds the floor of a short launch. Tiles of 64 queries (8 x 8
+// sums a lane, 13% fewer instructions) made those rounds twice as long: 160 us against
+// 136 for 16 heads of 64 below. One workgroup walking a tile's blocks one after the other
+// with 4 x 4 sums a thread (before) was bound by its LDS reads and barriers. Four
+// waves per SIMD (128 registers) spill and gain nothing. Measured on 3 sequences of
+// 861 rows, before and now: 16 heads of 64 244 -> 136 us, 4 heads of 128 287 -> 88 us;
+// of 100 rows 25.5 -> 21.6 and 38 -> 34 us; of 2,580 rows 1,222 -> 910 and 942 -> 494.
+template <int HW, int W, bool Rotary>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) void prefill_kernel(
     const uint16_t* __restrict__ qkv, int width, const int* __restrict__ sequence_start,
     const int* __restrict__ sequence_length, const int* __restrict__ sequence_replay,
     const uint16_t* __restrict__ rotations, int heads, float scale, uint16_t* __restrict__ out)
 {
-    constexpr int row = PrefillShared<HW>::row;
-    constexpr int columns = HW / 16;
-    __shared__ PrefillShared<HW> shared;
-    (void)heads; // the grid's z extent
-    const int sequence = blockIdx.x, head = blockIdx.z;
+    using Shared = PrefillShared<HW, W>;
+    constexpr int q_row = Shared::q_row, k_row = Shared::k_row, p_row = Shared::p_row;
+    __shared__ Shared shared;
+    const int sequence = blockIdx.x / heads, head = blockIdx.x % heads;
     const int length = sequence_length[sequence];
-    const int q0 = blockIdx.y * tile;
+    // The longest histories first.
+    const int q0 = int(gridDim.y - 1 - blockIdx.y) * queries;
     if (q0 >= length)
     {
         return;
     }
     const int replay = sequence_replay[sequence];
     const std::size_t stride = std::size_t(3) * width;
-    const uint16_t* base = qkv + std::size_t(sequence_start[sequence]) * stride + head * HW;
-    const int tid = threadIdx.x, group = tid / 16, slot = tid % 16;
+    const uint16_t* const base = qkv + std::size_t(sequence_start[sequence]) * stride + head * HW;
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x / 64));
+    const int lq = lane / 8, lk = lane % 8;
 
-    load_tile<HW>(shared.q, base, stride, q0, length, rotations);
-
-    float numerator[4][columns];
-    float running_maximum[4], total[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int i = threadIdx.x; i < queries * HW / 8; i += 64 * W)
     {
-        running_maximum[a] = -__builtin_inff();
-        total[a] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < columns; ++c)
+        const int r = i / (HW / 8), c = i % (HW / 8), position = q0 + r;
+        u32x4 u = u32x4{0, 0, 0, 0};
+        if (position < length)
         {
-            numerator[a][c] = 0.0f;
+            u = *reinterpret_cast<const u32x4*>(base + std::size_t(position) * stride + c * 8);
+            if constexpr (Rotary)
+            {
+                u = rotate8(u, load16(rotations + std::size_t(position) * HW + c * 8));
+            }
         }
+        *reinterpret_cast<u32x4*>(shared.q + r * q_row + c * 8) = u;
     }
-    const int last_block = (q0 + tile - 1 < length - 1 ? q0 + tile - 1 : length - 1) / tile;
-    for (int block = 0; block <= last_block; ++block)
+    // The state before the first block: original_exp(-inf) scales it away.
+    for (int i = threadIdx.x; i < HW / 64 * per_lane * 2 * 64; i += 64 * W)
+    {
+        shared.numerator[i / 64][i % 64] = f32x4{0, 0, 0, 0};
+    }
+    if (threadIdx.x < queries)
+    {
+        shared.maximum[threadIdx.x] = -__builtin_inff();
+        shared.total[threadIdx.x] = 0.0f;
+    }
+    if (threadIdx.x < HW / value_coordinates)
+    {
+        shared.turn[threadIdx.x] = 0;
+    }
+    __syncthreads();
+
+    typename Shared::Wave& mine = shared.wave[wave];
+    const int last_block = (q0 + queries - 1 < length - 1 ? q0 + queries - 1 : length - 1) / tile;
+    for (int block = wave; block <= last_block; block += W)
     {
         const int k0 = block * tile;
-        __syncthreads(); // previous block's K/V/P reads are done
-        if constexpr (wide_keys<HW>)
+        // Keys past the sequence read its last one, and are masked out.
+        u32x4 held[4], held_rotation[4] = {};
+        const auto fetch_keys = [&](int phase)
         {
-            load_tile<HW>(shared.kf, base + width, stride, k0, length, rotations);
-        }
-        else
-        {
-            load_tile<HW>(shared.k, base + width, stride, k0, length, rotations);
-        }
-        load_tile<HW>(shared.v, base + 2 * width, stride, k0, length, nullptr);
-        __syncthreads();
-
-        // Scores for 4 queries x 4 keys: serial fma chains over coordinates.
-        float dot[4][4];
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int j = 0; j < 4; ++j)
             {
-                dot[a][b] = 0.0f;
-            }
-        for (int c = 0; c < HW / 8; ++c)
-        {
-            uint4 qu[4], ku[4];
-            float4 kf[4][2];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-            {
-                qu[a] = *reinterpret_cast<const uint4*>(shared.q + (4 * group + a) * row + c * 8);
-                if constexpr (wide_keys<HW>)
+                const int i = lane + 64 * j, r = i / 4, c = phase * phase_coordinates + i % 4 * 8;
+                const int position = k0 + r < length ? k0 + r : length - 1;
+                held[j] = *reinterpret_cast<const u32x4*>(base + std::size_t(position) * stride + width + c);
+                if constexpr (Rotary)
                 {
-                    const float4* k = reinterpret_cast<const float4*>(
-                        shared.kf + (slot + 16 * a) * PrefillShared<HW>::key_row + c * 8);
-                    kf[a][0] = k[0];
-                    kf[a][1] = k[1];
-                }
-                else
-                {
-                    ku[a] = *reinterpret_cast<const uint4*>(shared.k + (slot + 16 * a) * row + c * 8);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-            {
-                float qv[4], kv[4];
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-                {
-                    const uint32_t qw[4] = {qu[a].x, qu[a].y, qu[a].z, qu[a].w};
-                    qv[a] = bf16_to_float(uint16_t(e % 2 ? qw[e / 2] >> 16 : qw[e / 2] & 0xffff));
-                    if constexpr (wide_keys<HW>)
-                    {
-                        const float4 h = kf[a][e / 4];
-                        const float k4[4] = {h.x, h.y, h.z, h.w};
-                        kv[a] = k4[e % 4];
-                    }
-                    else
-                    {
-                        const uint32_t kw[4] = {ku[a].x, ku[a].y, ku[a].z, ku[a].w};
-                        kv[a] = bf16_to_float(uint16_t(e % 2 ? kw[e / 2] >> 16 : kw[e / 2] & 0xffff));
-                    }
-                }
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b)
-                    {
-                        dot[a][b] = __builtin_fmaf(qv[a], kv[b], dot[a][b]);
-                    }
-            }
-        }
-        float block_maximum[4], block_sum[4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-        {
-            const int query = q0 + 4 * group + a;
-            float score[4];
-            float maximum = -__builtin_inff();
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-            {
-                const int key = k0 + slot + 16 * b;
-                const bool valid = key <= query && key < length;
-                score[b] = dot[a][b] * scale;
-                if (valid)
-                {
-                    maximum = maximum < score[b] ? score[b] : maximum;
-                }
-            }
-            maximum = group_max<16>(maximum);
-            float e[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-            {
-                const int key = k0 + slot + 16 * b;
-                const bool valid = key <= query && key < length;
-                e[b] = 0.0f;
-                if (valid)
-                {
-                    const float shifted = score[b] - maximum;
-                    e[b] = original_exp(shifted);
-                }
-                shared.p[4 * group + a][slot + 16 * b] = e[b];
-            }
-            // Pair tree over the 64 (zero-padded) block positions; for eight or
-            // fewer live positions the extra +0 levels leave the eight-wide tree
-            // unchanged (src/format/categorical.cpp:44-50).
-            float quarters[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-            {
-                quarters[b] = tree_sum<16>(e[b]);
-            }
-            block_sum[a] = register_tree(quarters);
-            block_maximum[a] = maximum;
-        }
-        __syncthreads();
-        // Value sums: serial fma over each query's live keys, ascending. Keys
-        // are the outer loop, so each value row read and widened serves the
-        // thread's four queries; a query's chain stops at its own last key.
-        int count[4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-        {
-            const int query = q0 + 4 * group + a;
-            const int live = (query < k0 + tile - 1 ? query : k0 + tile - 1) - k0 + 1;
-            count[a] = query >= length ? 0 : live < length - k0 ? live : length - k0;
-        }
-        // Queries past the sequence (count 0) are never merged, so they need
-        // not stop the others' unchecked loop.
-        int common = tile, most = 0;
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-        {
-            if (count[a] > 0)
-            {
-                common = min(common, count[a]);
-                most = max(most, count[a]);
-            }
-        }
-        common = min(common, most);
-        float sums[4][columns];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-        {
-#pragma unroll
-            for (int c = 0; c < columns; ++c)
-            {
-                sums[a][c] = 0.0f;
-            }
-        }
-        const auto accumulate = [&](int t, const float (&w)[4], bool every)
-        {
-            const uint16_t* vrow = shared.v + t * row + slot * columns;
-            float value[columns];
-#pragma unroll
-            for (int c = 0; c < columns; ++c)
-            {
-                value[c] = bf16_to_float(vrow[c]);
-            }
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-            {
-                if (every || t < count[a])
-                {
-#pragma unroll
-                    for (int c = 0; c < columns; ++c)
-                    {
-                        sums[a][c] = __builtin_fmaf(value[c], w[a], sums[a][c]);
-                    }
+                    held_rotation[j] = load16(rotations + std::size_t(position) * HW + c);
                 }
             }
         };
-        int t = 0;
-        for (; t + 4 <= common; t += 4)
-        {
-            float4 w4[4];
+        float dot[per_lane][8]; // scores, then weights
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < per_lane; ++a)
+        {
+#pragma unroll
+            for (int b = 0; b < 8; ++b)
             {
-                w4[a] = *reinterpret_cast<const float4*>(&shared.p[4 * group + a][t]);
+                dot[a][b] = 0.0f;
             }
-            accumulate(t, {w4[0].x, w4[1].x, w4[2].x, w4[3].x}, true);
-            accumulate(t + 1, {w4[0].y, w4[1].y, w4[2].y, w4[3].y}, true);
-            accumulate(t + 2, {w4[0].z, w4[1].z, w4[2].z, w4[3].z}, true);
-            accumulate(t + 3, {w4[0].w, w4[1].w, w4[2].w, w4[3].w}, true);
         }
-        for (; t < most; ++t)
+        for (int phase = 0; phase < HW / phase_coordinates; ++phase)
         {
-            accumulate(t, {shared.p[4 * group][t], shared.p[4 * group + 1][t], shared.p[4 * group + 2][t],
-                           shared.p[4 * group + 3][t]},
-                       false);
-        }
+            fetch_keys(phase);
+            tile_fence();
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-        {
-            const int query = q0 + 4 * group + a;
-            if (query >= length)
+            for (int j = 0; j < 4; ++j)
             {
-                continue;
+                const int i = lane + 64 * j, r = i / 4, c = i % 4;
+                *reinterpret_cast<u32x4*>(mine.k + r * k_row + c * 8) =
+                    Rotary ? rotate8(held[j], held_rotation[j]) : held[j];
             }
-            const bool round_values = query + 1 > 64 || query < replay;
-            const float maximum = block_maximum[a];
-            const float difference = maximum - running_maximum[a];
-            const float factor = original_exp(-__builtin_fabsf(difference));
-            const float old_scale = running_maximum[a] > maximum ? 1.0f : factor;
-            const float new_scale = running_maximum[a] > maximum ? factor : 1.0f;
-            const float old_total = total[a] * old_scale;
-            total[a] = __builtin_fmaf(block_sum[a], new_scale, old_total);
-#pragma unroll
-            for (int c = 0; c < columns; ++c)
+            tile_fence();
+#pragma unroll 1
+            for (int c = 0; c < phase_coordinates / 8; ++c)
             {
-                const float s = round_values ? round_bf16(sums[a][c]) : sums[a][c];
-                const float old = numerator[a][c] * old_scale;
-                numerator[a][c] = __builtin_fmaf(s, new_scale, old);
+                u32x4 qu[per_lane], ku[8];
+#pragma unroll
+                for (int a = 0; a < per_lane; ++a)
+                {
+                    qu[a] = *reinterpret_cast<const u32x4*>(shared.q + (lq + 8 * a) * q_row +
+                                                            phase * phase_coordinates + c * 8);
+                }
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+                {
+                    ku[b] = *reinterpret_cast<const u32x4*>(mine.k + (lk + 8 * b) * k_row + c * 8);
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                {
+                    float qv[per_lane], kv[8];
+#pragma unroll
+                    for (int a = 0; a < per_lane; ++a)
+                    {
+                        qv[a] = __uint_as_float(e % 2 ? qu[a][e / 2] & 0xffff0000u : qu[a][e / 2] << 16);
+                    }
+#pragma unroll
+                    for (int b = 0; b < 8; ++b)
+                    {
+                        kv[b] = __uint_as_float(e % 2 ? ku[b][e / 2] & 0xffff0000u : ku[b][e / 2] << 16);
+                    }
+#pragma unroll
+                    for (int a = 0; a < per_lane; ++a)
+                    {
+#pragma unroll
+                        for (int b = 0; b < 8; ++b)
+                        {
+                            dot[a][b] = __builtin_fmaf(qv[a], kv[b], dot[a][b]);
+                        }
+                    }
+                }
             }
-            running_maximum[a] = running_maximum[a] < maximum ? maximum : running_maximum[a];
         }
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-    {
-        const int query = q0 + 4 * group + a;
-        if (query >= length)
+
+        // Value rows, 16 keys x 64 coordinates at a time: rows past the sequence
+        // read its last one, and their weights are never applied.
+        u32x4 held_values[2];
+        const auto fetch_values = [&](int half, int chunk)
         {
-            continue;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+            {
+                const int i = lane + 64 * j, r = k0 + chunk * chunk_keys + i / 8;
+                const int position = r < length ? r : length - 1;
+                held_values[j] = *reinterpret_cast<const u32x4*>(base + std::size_t(position) * stride + 2 * width +
+                                                                 half * value_coordinates + i % 8 * 8);
+            }
+        };
+        fetch_values(0, 0);
+
+        // A query's last live key of the block (all of them but for the last block's).
+        int last_key[per_lane];
+#pragma unroll
+        for (int a = 0; a < per_lane; ++a)
+        {
+            const int query = q0 + lq + 8 * a;
+            last_key[a] = (query < length ? query : length - 1) - k0;
         }
-        const float reciprocal = 1.0f / total[a];
-        uint16_t* o = out + (std::size_t(sequence_start[sequence]) + query) * width + head * HW +
-                      slot * columns;
+        float block_maximum[per_lane], block_sum[per_lane];
+        // Whether every live score lies within 87 of its query's maximum. Then
+        // original_exp's clamps and its check change nothing, every weight is 0 or at
+        // least exp(-87) > 2^-126, so no sum of them is subnormal and the FTZ tree's
+        // flushes change nothing either.
+        bool ordinary = true;
 #pragma unroll
-        for (int c = 0; c < columns; ++c)
+        for (int a = 0; a < per_lane; ++a)
         {
-            o[c] = float_to_bf16(numerator[a][c] * reciprocal);
+            float maximum = -__builtin_inff();
+#pragma unroll
+            for (int b = 0; b < 8; ++b)
+            {
+                const float score = dot[a][b] * scale;
+                dot[a][b] = score;
+                const float live = lk + 8 * b <= last_key[a] ? score : -__builtin_inff();
+                maximum = maximum < live ? live : maximum;
+            }
+            maximum = group_max<8>(maximum);
+#pragma unroll
+            for (int b = 0; b < 8; ++b)
+            {
+                const float shifted = dot[a][b] - maximum;
+                dot[a][b] = shifted;
+                ordinary = ordinary & ((lk + 8 * b > last_key[a]) | (shifted >= -87.0f));
+            }
+            block_maximum[a] = maximum;
+        }
+        const bool plain = __all(ordinary);
+        // Pair tree over the 64 (zero-padded) block positions; for eight or fewer
+        // live positions the extra +0 levels leave the eight-wide tree unchanged
+        // (src/format/categorical.cpp:44-50).
+        const auto weigh = [&](auto exponential, auto tree)
+        {
+#pragma unroll
+            for (int a = 0; a < per_lane; ++a)
+            {
+                float eighths[8];
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+                {
+                    const float e = exponential(dot[a][b]);
+                    dot[a][b] = lk + 8 * b <= last_key[a] ? e : 0.0f;
+                    eighths[b] = dot[a][b];
+                }
+                block_sum[a] = tree(eighths);
+                // One query at a time, before the value rows are waited for: all
+                // eight at once would spill.
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+                {
+                    asm volatile("" : "+v"(dot[a][b]));
+                }
+                asm volatile("" : "+v"(block_sum[a]));
+            }
+        };
+        if (plain)
+        {
+            weigh([](float z) { return exp_within(z); },
+                  [](float (&v)[8])
+                  {
+#pragma unroll
+                      for (int b = 0; b < 8; ++b)
+                      {
+                          v[b] = plain_tree_sum<8>(v[b]);
+                      }
+                      return register_tree<8, false>(v);
+                  });
+        }
+        else
+        {
+            weigh([](float z) { return original_exp(z); },
+                  [](float (&v)[8])
+                  {
+#pragma unroll
+                      for (int b = 0; b < 8; ++b)
+                      {
+                          v[b] = tree_sum<8>(v[b]);
+                      }
+                      return register_tree(v);
+                  });
+        }
+
+        float old_scale[per_lane], new_scale[per_lane];
+#pragma unroll 1
+        for (int half = 0; half < HW / value_coordinates; ++half)
+        {
+            // Value sums: serial fma over each query's live keys, ascending. Dead
+            // keys have weight 0, and fma(value, 0, sum) leaves every sum but -0 as it
+            // is, unless the value is not finite; the sums of the last block (the only
+            // one with dead keys) are made again with those terms left out where one
+            // came out zero or NaN.
+            float sums[per_lane][8];
+            const int last_live = min(q0 + queries - 1, length - 1) - k0; // of any query
+            const auto accumulate = [&]<bool Careful>()
+            {
+#pragma unroll
+                for (int a = 0; a < per_lane; ++a)
+                {
+#pragma unroll
+                    for (int c = 0; c < 8; ++c)
+                    {
+                        sums[a][c] = 0.0f;
+                    }
+                }
+                if (Careful || half > 0)
+                {
+                    fetch_values(half, 0);
+                }
+#pragma unroll
+                for (int chunk = 0; chunk < tile / chunk_keys; ++chunk)
+                {
+                    if (chunk * chunk_keys > last_live)
+                    {
+                        break;
+                    }
+                    tile_fence();
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                    {
+                        const int b = chunk * 2 + i;
+                        *reinterpret_cast<f32x4*>(mine.p + (lk + 8 * i) * p_row + lq * 4) =
+                            f32x4{dot[0][b], dot[1][b], dot[2][b], dot[3][b]};
+                        *reinterpret_cast<u32x4*>(mine.v + (lane + 64 * i) * 8) = held_values[i];
+                    }
+                    tile_fence();
+                    if (chunk + 1 < tile / chunk_keys)
+                    {
+                        fetch_values(half, chunk + 1);
+                    }
+                    const auto term = [&](int t)
+                    {
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(mine.p + t * p_row + lq * 4);
+                        float value[8];
+                        widen8(*reinterpret_cast<const u32x4*>(mine.v + t * value_coordinates + lk * 8), value);
+#pragma unroll
+                        for (int a = 0; a < per_lane; ++a)
+                        {
+#pragma unroll
+                            for (int c = 0; c < 8; ++c)
+                            {
+                                const float next = __builtin_fmaf(value[c], w[a], sums[a][c]);
+                                sums[a][c] = !Careful || chunk * chunk_keys + t <= last_key[a] ? next : sums[a][c];
+                            }
+                        }
+                    };
+                    if constexpr (Careful)
+                    {
+#pragma unroll 1
+                        for (int t = 0; t < chunk_keys; ++t)
+                        {
+                            term(t);
+                        }
+                    }
+                    else
+                    {
+#pragma unroll 2
+                        for (int t = 0; t < chunk_keys; ++t)
+                        {
+                            term(t);
+                        }
+                    }
+                }
+            };
+            accumulate.template operator()<false>();
+            if (block == last_block)
+            {
+                bool settled = true;
+#pragma unroll
+                for (int a = 0; a < per_lane; ++a)
+                {
+#pragma unroll
+                    for (int c = 0; c < 8; ++c)
+                    {
+                        settled = settled & __builtin_islessgreater(sums[a][c], 0.0f);
+                    }
+                }
+                if (!__all(settled))
+                {
+                    accumulate.template operator()<true>();
+                }
+            }
+
+            // The running state up to this block.
+            while (__hip_atomic_load(&shared.turn[half], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != block)
+            {
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (half == 0)
+            {
+#pragma unroll
+                for (int a = 0; a < per_lane; ++a)
+                {
+                    const int q = lq + 8 * a;
+                    const float running = shared.maximum[q];
+                    const float total = shared.total[q];
+                    const float maximum = block_maximum[a];
+                    const float factor = original_exp(-__builtin_fabsf(maximum - running));
+                    old_scale[a] = running > maximum ? 1.0f : factor;
+                    new_scale[a] = running > maximum ? factor : 1.0f;
+                    const float old_total = total * old_scale[a];
+                    block_sum[a] = __builtin_fmaf(block_sum[a], new_scale[a], old_total);
+                    block_maximum[a] = running < maximum ? maximum : running;
+                }
+                tile_fence(); // every lane has read the row its own lanes now write
+#pragma unroll
+                for (int a = 0; a < per_lane; ++a)
+                {
+                    shared.maximum[lq + 8 * a] = block_maximum[a];
+                    shared.total[lq + 8 * a] = block_sum[a];
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < per_lane; ++a)
+            {
+                const int query = q0 + lq + 8 * a;
+                const bool round_values = query + 1 > 64 || query < replay;
+                float numerator[8];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                {
+                    const f32x4 n = shared.numerator[(half * per_lane + a) * 2 + h][lane];
+                    const float old4[4] = {n.x, n.y, n.z, n.w};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        const int c = h * 4 + i;
+                        const float sum = round_values ? round_bf16(sums[a][c]) : sums[a][c];
+                        const float old = old4[i] * old_scale[a];
+                        numerator[c] = __builtin_fmaf(sum, new_scale[a], old);
+                    }
+                }
+                if (block < last_block)
+                {
+                    shared.numerator[(half * per_lane + a) * 2][lane] =
+                        f32x4{numerator[0], numerator[1], numerator[2], numerator[3]};
+                    shared.numerator[(half * per_lane + a) * 2 + 1][lane] =
+                        f32x4{numerator[4], numerator[5], numerator[6], numerator[7]};
+                }
+                else if (query < length)
+                {
+                    const float reciprocal = 1.0f / block_sum[a];
+                    uint32_t words[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        words[i] = float_to_bf16(numerator[2 * i] * reciprocal) |
+                                   (uint32_t(float_to_bf16(numerator[2 * i + 1] * reciprocal)) << 16);
+                    }
+                    __builtin_memcpy(out + (std::size_t(sequence_start[sequence]) + query) * width + head * HW +
+                                         half * value_coordinates + lk * 8,
+                                     words, 16);
+                }
+            }
+            if (lane == 0)
+            {
+                __hip_atomic_store(&shared.turn[half], block + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
         }
     }
 }
@@ -878,20 +1040,30 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     {
         return;
     }
-    const dim3 grid(unsigned(sequences), unsigned((max_length + tile - 1) / tile), unsigned(heads));
-    switch (head_width)
+    require(head_width == 64 || head_width == 128, "attention: head width must be 64 or 128");
+    require(sequences * heads < (std::size_t(1) << 31), "attention: too many sequences");
+    const dim3 grid(unsigned(sequences * heads), unsigned((max_length + queries - 1) / queries));
+    const auto launch = [&](auto rotary, auto plain, int waves)
     {
-    case 64:
-        prefill_kernel<64><<<grid, 256, 0, stream>>>(qkv, int(width), sequence_start, sequence_length,
-                                                     sequence_replay, rotations, int(heads), scale, out);
-        break;
-    case 128:
-        prefill_kernel<128><<<grid, 256, 0, stream>>>(qkv, int(width), sequence_start,
-                                                      sequence_length, sequence_replay, rotations,
-                                                      int(heads), scale, out);
-        break;
-    default:
-        throw Error("attention: head width must be 64 or 128");
+        (rotations ? rotary : plain)<<<grid, 64 * waves, 0, stream>>>(qkv, int(width), sequence_start, sequence_length, sequence_replay,
+                                                rotations, int(heads), scale, out);
+    };
+    // Eight waves take twice the blocks of a query tile at a time, which pays only
+    // where histories have more than four blocks and the grid alone does not fill the
+    // device (16 heads of 64, 4 against 8 waves: one sequence of 862 rows, 432
+    // workgroups, 75 and 63 us; three of 430, 672 workgroups, 53 and 70 us; 4 heads of
+    // 128, three of 861, 324 workgroups, 133 and 88 us).
+    const bool eight =
+        max_length > 4 * tile && std::size_t(grid.x) * grid.y < 2 * std::size_t(compute_units());
+    if (head_width == 64)
+    {
+        eight ? launch(prefill_kernel<64, 8, true>, prefill_kernel<64, 8, false>, 8)
+              : launch(prefill_kernel<64, 4, true>, prefill_kernel<64, 4, false>, 4);
+    }
+    else
+    {
+        eight ? launch(prefill_kernel<128, 8, true>, prefill_kernel<128, 8, false>, 8)
+              : launch(prefill_kernel<128, 4, true>, prefill_kernel<128, 4, false>, 4);
     }
     check_hip(hipGetLastError(), "attention prefill launch");
 }

@@ -775,22 +775,6 @@ void dac_conv_layout(const ConvShape& s, const float* stored, float* out, int co
     }
 }
 
-namespace
-{
-int compute_units()
-{
-    static const int count = []
-    {
-        int device = 0, units = 0;
-        check_hip(hipGetDevice(&device), "hipGetDevice");
-        check_hip(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device),
-                  "hipDeviceGetAttribute");
-        return units > 0 ? units : 1;
-    }();
-    return count;
-}
-} // namespace
-
 void dac_conv(const ConvArgs& a, hipStream_t stream)
 {
     const ConvShape& s = a.conv.shape;

@@ -85,6 +85,25 @@ __device__ __forceinline__ float original_exp(float z)
     return __uint_as_float(__float_as_uint(plus_one) + (uint32_t(n) << 23));
 }
 
+// original_exp for z in [-87, 87], where its clamps and its check of the exponent
+// leave z and n as they are.
+__device__ __forceinline__ float exp_within(float z)
+{
+    const float exponent = z * 0x1.715476p+0f;
+    const int32_t n = int32_t(__builtin_rintf(exponent));
+    z = __builtin_fmaf(float(n), -0x1.630000p-1f, z);
+    z = __builtin_fmaf(float(n), 0x1.bd0106p-13f, z);
+    float p = __builtin_fmaf(0x1.a01a02p-13f, z, 0x1.6c16c2p-10f);
+    p = __builtin_fmaf(p, z, 0x1.111112p-7f);
+    p = __builtin_fmaf(p, z, 0x1.555556p-5f);
+    p = __builtin_fmaf(p, z, 0x1.555556p-3f);
+    const float square = z * z;
+    p = __builtin_fmaf(p, z, 0.5f);
+    z = __builtin_fmaf(p, square, z);
+    const float plus_one = z + 1.0f;
+    return __uint_as_float(__float_as_uint(plus_one) + (uint32_t(n) << 23));
+}
+
 // tanh-GELU with the reference's rounding boundaries (src/common/probability.cpp:45-63).
 __device__ __forceinline__ uint16_t gelu_bf16(uint16_t bits)
 {

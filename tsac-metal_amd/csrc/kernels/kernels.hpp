@@ -33,6 +33,20 @@ inline void check_hip(hipError_t status, const char* what)
     }
 }
 
+// Compute units of the device current at the first call.
+inline int compute_units()
+{
+    static const int count = []
+    {
+        int device = 0, units = 0;
+        check_hip(hipGetDevice(&device), "hipGetDevice");
+        check_hip(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device),
+                  "hipDeviceGetAttribute");
+        return units > 0 ? units : 1;
+    }();
+    return count;
+}
+
 // Error words written by kernels (plain stores of fixed values):
 // word 0 = a BF8L, softmax or categorical input was not finite; word 1 = the
 // range decoder failed; word 2 = a frame-step wait stalled (see frame.hpp).

@@ -690,20 +690,6 @@ __global__ __launch_bounds__(gemm::threads, Cfg::per_cu) void gemm_kernel(
                 }
     }
 }
-
-int compute_units()
-{
-    static const int count = []
-    {
-        int device = 0, units = 0;
-        check_hip(hipGetDevice(&device), "hipGetDevice");
-        check_hip(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device),
-                  "hipDeviceGetAttribute");
-        return units > 0 ? units : 1;
-    }();
-    return count;
-}
-
 template <class Cfg>
 void launch_gemm_config(const DeviceLinear& w, const int8_t* q, const float* scales, std::size_t M, uint16_t* y,
                         const uint16_t* residual, Layout layout, hipStream_t stream)
