@@ -550,7 +550,8 @@ def test_calibration_probes(torch, native):
 
 @pytest.mark.parametrize("heads,hw", [(16, 64), (4, 128)])
 @pytest.mark.parametrize("lengths,kind", [([65, 31, 33, 64, 1] * 8, "normal"), ([330], "normal"), ([129, 96], "spread"),
-                                          ([100], "dead infinity"), ([70], "zeros"), ([65], "tiny")])
+                                          ([100], "dead infinity"), ([70], "zeros"), ([65], "tiny"), ([12] * 9, "normal"),
+                                          ([1, 16, 15, 2, 7], "spread"), ([9, 16], "zeros"), ([16], "tiny")])
 def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, kind):
     """The causal kernel's own choices: 4 or 8 waves by the grid, edges of its 32-query
     and 64-key tiles, scores more than 87 below the maximum (where weights and their

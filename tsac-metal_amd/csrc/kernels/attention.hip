@@ -934,6 +934,182 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
         }
     }
 }
+
+// Sequences of at most 16 rows (the codebook stack's: a frame's books), one wave per
+// (sequence, head). Lane (g, t) = (lane / 16, lane % 16) holds the scores of key t
+// with queries g + 4 a, so the 16-lane butterfly is the pair tree over the block (its
+// higher levels add +0); then lane l holds the value sums of coordinates l (64-wide
+// heads) or 2 l and 2 l + 1 of every query. There is one block, merged into the
+// empty state by the recurrence all the same.
+//
+// Bound by HBM: each row of the projection is read once and each output written once.
+// 2,580 sequences of 12 rows, 16 heads of 64 (253 MB): 638 us on the tiled kernel above,
+// whose waves each take a whole 64-key block, 85 here (3.0 TB/s); 4 heads of 128, 39.
+constexpr int short_rows = 16, short_waves = 4;
+
+template <int HW, bool Rotary>
+__global__ __launch_bounds__(64 * short_waves) void short_kernel(
+    const uint16_t* __restrict__ qkv, int width, const int* __restrict__ sequence_start,
+    const int* __restrict__ sequence_length, const int* __restrict__ sequence_replay,
+    const uint16_t* __restrict__ rotations, int heads, int pairs, float scale, uint16_t* __restrict__ out)
+{
+    constexpr int row = HW + 8, chunks = HW / 8, columns = HW / 64;
+    constexpr int loads = short_rows * chunks / 64;
+    __shared__ __attribute__((aligned(16))) uint16_t tiles[short_waves][2][short_rows * row];
+    __shared__ __attribute__((aligned(16))) float weights[short_waves][short_rows][short_rows + 4];
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x / 64));
+    const int pair = int(blockIdx.x) * short_waves + wave;
+    if (pair >= pairs)
+    {
+        return;
+    }
+    const int sequence = pair / heads, head = pair % heads;
+    const int length = min(sequence_length[sequence], short_rows);
+    if (length <= 0)
+    {
+        return;
+    }
+    const int replay = sequence_replay[sequence];
+    const std::size_t stride = std::size_t(3) * width;
+    const std::size_t first = std::size_t(sequence_start[sequence]);
+    const uint16_t* const base = qkv + first * stride + head * HW;
+    uint16_t* const query_tile = tiles[wave][0];
+    uint16_t* const key_tile = tiles[wave][1];
+
+    // Rows past the sequence repeat its last one, and are masked out or not stored.
+    u32x4 held[2][loads], held_rotation[loads] = {};
+#pragma unroll
+    for (int j = 0; j < loads; ++j)
+    {
+        const int i = lane + 64 * j, r = i / chunks, c = i % chunks * 8;
+        const int position = r < length ? r : length - 1;
+        const uint16_t* const from = base + std::size_t(position) * stride + c;
+        held[0][j] = *reinterpret_cast<const u32x4*>(from);
+        held[1][j] = *reinterpret_cast<const u32x4*>(from + width);
+        if constexpr (Rotary)
+        {
+            held_rotation[j] = load16(rotations + std::size_t(position) * HW + c);
+        }
+    }
+    uint32_t values[short_rows]; // the lane's coordinates of each row, BF16
+#pragma unroll
+    for (int t = 0; t < short_rows; ++t)
+    {
+        const uint16_t* const from =
+            base + std::size_t(t < length ? t : length - 1) * stride + 2 * width + columns * lane;
+        if constexpr (columns == 2)
+        {
+            __builtin_memcpy(&values[t], from, 4);
+        }
+        else
+        {
+            values[t] = *from;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < loads; ++j)
+    {
+        const int i = lane + 64 * j, r = i / chunks, c = i % chunks * 8;
+        *reinterpret_cast<u32x4*>(query_tile + r * row + c) =
+            Rotary ? rotate8(held[0][j], held_rotation[j]) : held[0][j];
+        *reinterpret_cast<u32x4*>(key_tile + r * row + c) =
+            Rotary ? rotate8(held[1][j], held_rotation[j]) : held[1][j];
+    }
+    tile_fence();
+
+    const int g = lane / 16, t = lane % 16;
+    float dot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int c = 0; c < chunks; ++c)
+    {
+        float kv[8], qv[8];
+        widen8(*reinterpret_cast<const u32x4*>(key_tile + t * row + c * 8), kv);
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+        {
+            widen8(*reinterpret_cast<const u32x4*>(query_tile + (g + 4 * a) * row + c * 8), qv);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+            {
+                dot[a] = __builtin_fmaf(qv[e], kv[e], dot[a]);
+            }
+        }
+    }
+    // Each query's weights, and the scales its block joins the empty state with.
+    float total[4], old_scale[4], new_scale[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+    {
+        const int query = g + 4 * a;
+        const bool live = t <= query && t < length;
+        const float score = dot[a] * scale;
+        float maximum = -__builtin_inff();
+        maximum = live && maximum < score ? score : maximum;
+        maximum = group_max<16>(maximum);
+        const float e = original_exp(score - maximum);
+        const float weight = live ? e : 0.0f;
+        weights[wave][query][t] = weight;
+        const float sum = tree_sum<16>(weight);
+        const float running = -__builtin_inff();
+        const float factor = original_exp(-__builtin_fabsf(maximum - running));
+        old_scale[a] = running > maximum ? 1.0f : factor;
+        new_scale[a] = running > maximum ? factor : 1.0f;
+        total[a] = __builtin_fmaf(sum, new_scale[a], 0.0f * old_scale[a]);
+    }
+    tile_fence();
+#pragma unroll
+    for (int query = 0; query < short_rows; ++query)
+    {
+        if (query >= length)
+        {
+            continue;
+        }
+        // From a lane of the query's group.
+        const int source = query % 4 * 16;
+        const float query_total = __shfl(total[query / 4], source), query_old = __shfl(old_scale[query / 4], source),
+                    query_new = __shfl(new_scale[query / 4], source);
+        float sums[columns];
+#pragma unroll
+        for (int c = 0; c < columns; ++c)
+        {
+            sums[c] = 0.0f;
+        }
+        // Serial fma over the query's live keys, ascending.
+#pragma unroll
+        for (int key = 0; key < short_rows; ++key)
+        {
+            if (key > query)
+            {
+                continue;
+            }
+            const float weight = weights[wave][query][key];
+#pragma unroll
+            for (int c = 0; c < columns; ++c)
+            {
+                const float value = __uint_as_float(c ? values[key] & 0xffff0000u : values[key] << 16);
+                sums[c] = __builtin_fmaf(value, weight, sums[c]);
+            }
+        }
+        const float reciprocal = 1.0f / query_total;
+        uint32_t word = 0;
+#pragma unroll
+        for (int c = 0; c < columns; ++c)
+        {
+            const float sum = query < replay ? round_bf16(sums[c]) : sums[c];
+            const float numerator = __builtin_fmaf(sum, query_new, 0.0f * query_old);
+            word |= uint32_t(float_to_bf16(numerator * reciprocal)) << (16 * c);
+        }
+        uint16_t* const to = out + (first + query) * width + head * HW + columns * lane;
+        if constexpr (columns == 2)
+        {
+            __builtin_memcpy(to, &word, 4);
+        }
+        else
+        {
+            *to = uint16_t(word);
+        }
+    }
+}
 } // namespace
 
 void append_qkv(const uint16_t* qkv, std::size_t rows, std::size_t width, std::size_t head_width,
@@ -1042,6 +1218,17 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     }
     require(head_width == 64 || head_width == 128, "attention: head width must be 64 or 128");
     require(sequences * heads < (std::size_t(1) << 31), "attention: too many sequences");
+    if (max_length <= short_rows)
+    {
+        const std::size_t pairs = sequences * heads;
+        const auto kernel = head_width == 64 ? (rotations ? short_kernel<64, true> : short_kernel<64, false>)
+                                             : (rotations ? short_kernel<128, true> : short_kernel<128, false>);
+        kernel<<<unsigned((pairs + short_waves - 1) / short_waves), 64 * short_waves, 0, stream>>>(
+            qkv, int(width), sequence_start, sequence_length, sequence_replay, rotations, int(heads), int(pairs), scale,
+            out);
+        check_hip(hipGetLastError(), "attention prefill launch");
+        return;
+    }
     const dim3 grid(unsigned(sequences * heads), unsigned((max_length + queries - 1) / queries));
     const auto launch = [&](auto rotary, auto plain, int waves)
     {
