@@ -690,55 +690,72 @@ std::vector<uint8_t> Session::encode(Header h, const uint16_t* tokens, std::size
     validate(h, tokens, count);
     require(model_->limits().file_bytes >= 19, "the stream limit is below the 19-byte FBAZ framing");
     const uint32_t crc = token_crc32(tokens, count);
-    std::vector<uint16_t> splits(count * 16);
+    // Page-locked up to 16 MiB (some eight minutes of stereo), where the copy from the
+    // device is one transfer.
+    constexpr std::size_t staged = std::size_t(16) << 20;
+    std::vector<uint16_t> unstaged;
+    uint16_t* splits = nullptr;
+    if (count * 32 <= staged)
+    {
+        staging_splits_.reserve(std::max<std::size_t>(count, 1) * 32);
+        splits = staging_splits_.as<uint16_t>();
+    }
+    else
+    {
+        unstaged.resize(count * 16);
+        splits = unstaged.data();
+    }
     reset_errors();
     const KnownPlan plan = plan_known(h);
     frame_launch_ = -1;
     if (plan.stepwise)
     {
-        stepwise(h, tokens, nullptr, 0, nullptr, nullptr, splits.data());
+        stepwise(h, tokens, nullptr, 0, nullptr, nullptr, splits);
     }
     else
     {
-        batched(h, tokens, nullptr, splits.data(), plan);
+        batched(h, tokens, nullptr, splits, plan);
     }
     check_errors();
     const double t1 = now();
     // Host range coding in stream order (src/format/entropy.cpp:57-100): the ten
     // Q15 splits along each symbol's bisection path, computed on the GPU.
-    RangeEncoder encoder(model_->limits().file_bytes - 18);
+    const std::size_t most = model_->limits().file_bytes - 18;
     const bool before = observer && observer->before, after = observer && observer->after;
-    for_each_position(h, [&](const Position& p)
+    std::vector<uint8_t> payload;
+    bool coded = false;
+    if (!before && !after)
     {
-        if (before)
+        SymbolEncoder encoder(count);
+        for_each_position(h, [&](const Position& p) { encoder.put(splits + p.offset * 16, tokens[p.offset]); });
+        payload = encoder.finish();
+        coded = payload.size() <= most;
+    }
+    if (!coded)
+    {
+        // For an observer, symbol by symbol; and for the error of a payload past the limit.
+        RangeEncoder encoder(most);
+        for_each_position(h, [&](const Position& p)
         {
-            observer->before(p);
-        }
-        const std::size_t start = after ? encoder.bit_position() : 0;
-        const uint16_t symbol = tokens[p.offset];
-        const uint16_t* s = splits.data() + p.offset * 16;
-        std::size_t base = 0, n = 1024;
-        for (int level = 0; n > 1; ++level)
-        {
-            const std::size_t half = n / 2;
-            const bool one = symbol >= base + half;
-            encoder.put(s[level], one);
-            if (one)
+            if (before)
             {
-                base += half;
-                n -= half;
+                observer->before(p);
             }
-            else
+            const std::size_t start = after ? encoder.bit_position() : 0;
+            const uint16_t symbol = tokens[p.offset];
+            const uint16_t* s = splits + p.offset * 16;
+            for (int level = 0; level < 10; ++level)
             {
-                n = half;
+                encoder.put(s[level], symbol >> (9 - level) & 1);
             }
-        }
-        if (after)
-        {
-            observer->after(p, encoder.bit_position() - start);
-        }
-    });
-    const auto bytes = frame_normal(h, crc, encoder.finish());
+            if (after)
+            {
+                observer->after(p, encoder.bit_position() - start);
+            }
+        });
+        payload = encoder.finish();
+    }
+    const auto bytes = frame_normal(h, crc, payload);
     const double t2 = now();
     timing_ = {t1 - t0, t2 - t1, t2 - t0, input_seconds(), 0.0, 0.0, double(frame_launch_),
                plan.stepwise ? 1.0 : 0.0};

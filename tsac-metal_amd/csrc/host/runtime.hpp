@@ -294,7 +294,7 @@ private:
     hipStream_t stream_ = nullptr;
     Arena arena_;
     DeviceBuffer errors_;
-    PinnedBuffer pinned_errors_, staging_, staging_nodes_, staging_tokens_;
+    PinnedBuffer pinned_errors_, staging_splits_, staging_, staging_nodes_, staging_tokens_;
     std::array<double, 8> timing_{};
     // TSAC_HIP_FRAME_LAUNCH=plain in the environment when the session was
     // created: frame steps go out as plain launches (see FrameArgs::plain_launch).
