@@ -585,3 +585,26 @@ def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, ki
             finite = np.isfinite(bf16_float(expected))
             assert np.array_equal(got[start + t][finite], expected[finite]), (length, t)
             assert not np.isfinite(bf16_float(got[start + t][~finite])).any()
+
+
+@pytest.mark.parametrize("k", [256, 512, 1024, 2048, 4096])
+@pytest.mark.parametrize("columns", range(1, 9))
+def test_qlinear_quantises_in_the_gemv(torch, native, oracle, k, columns):
+    """Up to 8 rows the projection quantises inside the GEMV; where the output overlaps
+    the input it takes two launches, and an output over the input must still be made
+    from the input as it was. A nonfinite input fails, and the next call does not."""
+    rng = np.random.default_rng(k + columns)
+    values, scales, bias = random_linear(rng, k, k)
+    linear = native.DeviceLinear(values, scales, bias)
+    x = _activations(rng, columns, k)
+    x[0, :256] = 0
+    expected = oracle.qlinear(values, scales, bias, x)
+    dx, y = dev(torch, x), empty(torch, (columns, k), torch.int16)
+    linear.apply(dx, y)
+    assert np.array_equal(host(y), expected)
+    bad = x.copy()
+    bad[columns - 1, k - 1] = 0x7F80
+    with pytest.raises(native.HipError, match="finite"):
+        linear.apply(dev(torch, bad), y)
+    linear.apply(dx, dx)
+    assert np.array_equal(host(dx), expected)

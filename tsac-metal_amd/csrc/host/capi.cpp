@@ -136,6 +136,207 @@ struct AsyncScratch
     }
 };
 
+// Device buffers for the projections' quantised activations, kept between calls: a
+// call waits for its stream before it returns, so a buffer given back is idle and
+// serves any stream and thread. (hipMallocAsync's pool maps its memory again after each
+// synchronisation, a release threshold or not: a 30,960-row block spent 300 us between
+// two kernels on it.) At most `kept` bytes a device stay; the last projection
+// destroyed frees them.
+class ProjectionBuffers
+{
+  public:
+    static constexpr std::size_t kept = std::size_t(512) << 20;
+
+    struct Buffer
+    {
+        void* pointer = nullptr;
+        std::size_t bytes = 0;
+        int device = 0;
+    };
+
+    // The smallest unused buffer of at least `bytes`, or a new one.
+    Buffer take(std::size_t bytes)
+    {
+        Buffer b;
+        check_hip(hipGetDevice(&b.device), "hipGetDevice");
+        {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            auto& unused = unused_[b.device];
+            auto found = unused.lower_bound(bytes);
+            if (found != unused.end())
+            {
+                b.bytes = found->first;
+                b.pointer = found->second;
+                unused.erase(found);
+                return b;
+            }
+        }
+        b.bytes = (bytes + 0xffff) / 0x10000 * 0x10000;
+        check_hip(hipMalloc(&b.pointer, b.bytes), "hipMalloc");
+        return b;
+    }
+    // Keeps an idle buffer, freeing the smallest ones beyond the bound.
+    void give(const Buffer& b)
+    {
+        std::vector<void*> freed;
+        {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            auto& unused = unused_[b.device];
+            unused.emplace(b.bytes, b.pointer);
+            std::size_t total = 0;
+            for (const auto& [bytes, pointer] : unused)
+            {
+                total += bytes;
+            }
+            while (total > kept || (!projections_ && !unused.empty()))
+            {
+                total -= unused.begin()->first;
+                freed.push_back(unused.begin()->second);
+                unused.erase(unused.begin());
+            }
+        }
+        for (void* p : freed)
+        {
+            (void)hipFree(p);
+        }
+    }
+    void created()
+    {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        ++projections_;
+    }
+    void destroyed()
+    {
+        std::vector<void*> freed;
+        {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            if (--projections_ == 0)
+            {
+                for (auto& [device, unused] : unused_)
+                {
+                    for (const auto& [bytes, pointer] : unused)
+                    {
+                        freed.push_back(pointer);
+                    }
+                }
+                unused_.clear();
+            }
+        }
+        for (void* p : freed)
+        {
+            (void)hipFree(p);
+        }
+    }
+
+  private:
+    std::mutex mutex_;
+    std::map<int, std::multimap<std::size_t, void*>> unused_;
+    std::size_t projections_ = 0;
+};
+
+ProjectionBuffers& projection_buffers()
+{
+    static auto* const buffers = new ProjectionBuffers; // outlives every thread's calls
+    return *buffers;
+}
+
+// The error words of one call, in page-locked host memory that its kernels store to:
+// nothing to clear on the device or to copy back. Words are reused; a block of 64
+// pairs is added where more calls overlap.
+class ErrorWords
+{
+  public:
+    explicit ErrorWords(hipStream_t stream) : stream_(stream)
+    {
+        const std::lock_guard<std::mutex> lock(mutex());
+        auto& words = unused();
+        if (words.empty())
+        {
+            void* block = nullptr;
+            check_hip(hipHostMalloc(&block, 64 * 64, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
+            words.reserve(words.capacity() + 64);
+            for (int i = 0; i < 64; ++i)
+            {
+                words.push_back(static_cast<uint32_t*>(block) + 16 * i);
+            }
+        }
+        host_ = words.back();
+        words.pop_back();
+        host_[0] = host_[1] = 0;
+    }
+    ~ErrorWords()
+    {
+        wait();
+        const std::lock_guard<std::mutex> lock(mutex());
+        unused().push_back(host_);
+    }
+    ErrorWords(const ErrorWords&) = delete;
+    ErrorWords& operator=(const ErrorWords&) = delete;
+
+    uint32_t* device() const
+    {
+        void* p = nullptr;
+        check_hip(hipHostGetDevicePointer(&p, host_, 0), "hipHostGetDevicePointer");
+        return static_cast<uint32_t*>(p);
+    }
+    // Waits for a call that failed on the way: its kernels may still be running.
+    void wait() const
+    {
+        if (!waited_)
+        {
+            (void)hipStreamSynchronize(stream_);
+        }
+    }
+    // Waits for the call's kernels and fails with `message` if one set its word.
+    void check(const char* message)
+    {
+        check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+        waited_ = true;
+        require(!*static_cast<volatile uint32_t*>(host_), message);
+    }
+
+  private:
+    static std::mutex& mutex()
+    {
+        static std::mutex* const m = new std::mutex;
+        return *m;
+    }
+    static std::vector<uint32_t*>& unused()
+    {
+        static auto* const words = new std::vector<uint32_t*>;
+        return *words;
+    }
+    uint32_t* host_ = nullptr;
+    hipStream_t stream_;
+    bool waited_ = false;
+};
+
+// One call's buffer; declared after its ErrorWords, whose check() has waited for the
+// stream unless the call failed.
+class ProjectionScratch
+{
+  public:
+    ProjectionScratch(std::size_t bytes, const ErrorWords& words)
+        : buffer_(projection_buffers().take(bytes)), words_(words)
+    {
+    }
+    ~ProjectionScratch()
+    {
+        words_.wait();
+        projection_buffers().give(buffer_);
+    }
+    ProjectionScratch(const ProjectionScratch&) = delete;
+    ProjectionScratch& operator=(const ProjectionScratch&) = delete;
+    void* get() const
+    {
+        return buffer_.pointer;
+    }
+
+  private:
+    ProjectionBuffers::Buffer buffer_;
+    const ErrorWords& words_;
+};
+
 // Decode-attention scratch kept per (device, stream): arrival counters at
 // the start, block records after them. The kernel leaves its counters at
 // zero, so they are cleared when allocated and then serve every later call on
@@ -826,13 +1027,18 @@ int tsac_hip_linear_create(const tsac_hip_linear* weights, size_t K, size_t N,
                       "upload");
             l->linear = {l->values.as<int8_t>(), reinterpret_cast<const float*>(c),
                          reinterpret_cast<const float*>(c + (scale_bytes + 255) / 256 * 256), K, N};
+            projection_buffers().created();
             *linear = l.release();
         });
 }
 
 void tsac_hip_linear_destroy(tsac_hip_device_linear* linear)
 {
-    delete linear;
+    if (linear)
+    {
+        delete linear;
+        projection_buffers().destroyed();
+    }
 }
 
 int tsac_hip_linear_apply(const tsac_hip_device_linear* linear, const uint16_t* x, size_t M,
@@ -851,18 +1057,19 @@ int tsac_hip_linear_apply(const tsac_hip_device_linear* linear, const uint16_t* 
                                 !small_gemm_chosen(M, linear->linear.N, K));
             const Layout layout = tiles ? Layout::tiles : Layout::rows;
             const std::size_t rows = tiles ? tile_padded_rows(M) : M;
-            AsyncScratch scratch(rows * K + rows * (K / 256) * 4 + 256 + 8, s);
-            auto* q = static_cast<int8_t*>(scratch.pointer);
+            ErrorWords errors(s);
+            if (quantizing_linear(linear->linear, x, M, y, chosen, errors.device(), s))
+            {
+                errors.check("BF8L activations must be finite");
+                return;
+            }
+            ProjectionScratch scratch(rows * K + rows * (K / 256) * 4 + 256, errors);
+            auto* q = static_cast<int8_t*>(scratch.get());
             auto* scales =
-                reinterpret_cast<float*>(static_cast<uint8_t*>(scratch.pointer) + (rows * K + 255) / 256 * 256);
-            auto* error = reinterpret_cast<uint32_t*>(scales + rows * (K / 256));
-            check_hip(hipMemsetAsync(error, 0, 8, s), "hipMemsetAsync");
-            quantize_rows(x, M, K, Prologue::none, nullptr, nullptr, q, scales, nullptr, error, s, layout);
+                reinterpret_cast<float*>(static_cast<uint8_t*>(scratch.get()) + (rows * K + 255) / 256 * 256);
+            quantize_rows(x, M, K, Prologue::none, nullptr, nullptr, q, scales, nullptr, errors.device(), s, layout);
             tsac_hip::linear(linear->linear, q, scales, M, y, nullptr, chosen, s, layout);
-            uint32_t flags[2];
-            check_hip(hipMemcpyAsync(flags, error, 8, hipMemcpyDeviceToHost, s), "read error words");
-            check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-            require(!flags[0], "BF8L activations must be finite");
+            errors.check("BF8L activations must be finite");
         });
 }
 
@@ -901,14 +1108,9 @@ int tsac_hip_bf8l(const uint16_t* x, size_t rows, size_t K, int8_t* q, float* sc
         [&]
         {
             const auto s = as_stream(stream);
-            AsyncScratch scratch(8, s);
-            auto* error = static_cast<uint32_t*>(scratch.pointer);
-            check_hip(hipMemsetAsync(error, 0, 8, s), "hipMemsetAsync");
-            quantize_rows(x, rows, K, Prologue::none, nullptr, nullptr, q, scales, nullptr, error, s);
-            uint32_t flags[2];
-            check_hip(hipMemcpyAsync(flags, error, 8, hipMemcpyDeviceToHost, s), "read error words");
-            check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-            require(!flags[0], "BF8L activations must be finite");
+            ErrorWords errors(s);
+            quantize_rows(x, rows, K, Prologue::none, nullptr, nullptr, q, scales, nullptr, errors.device(), s);
+            errors.check("BF8L activations must be finite");
         });
 }
 
@@ -918,15 +1120,10 @@ int tsac_hip_bf8l_tiles(const uint16_t* x, size_t rows, size_t K, int8_t* q, flo
         [&]
         {
             const auto s = as_stream(stream);
-            AsyncScratch scratch(8, s);
-            auto* error = static_cast<uint32_t*>(scratch.pointer);
-            check_hip(hipMemsetAsync(error, 0, 8, s), "hipMemsetAsync");
-            quantize_rows(x, rows, K, Prologue::none, nullptr, nullptr, q, scales, nullptr, error, s,
+            ErrorWords errors(s);
+            quantize_rows(x, rows, K, Prologue::none, nullptr, nullptr, q, scales, nullptr, errors.device(), s,
                           Layout::tiles);
-            uint32_t flags[2];
-            check_hip(hipMemcpyAsync(flags, error, 8, hipMemcpyDeviceToHost, s), "read error words");
-            check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-            require(!flags[0], "BF8L activations must be finite");
+            errors.check("BF8L activations must be finite");
         });
 }
 
@@ -947,14 +1144,9 @@ int tsac_hip_softmax(const uint16_t* x, size_t rows, size_t width, uint16_t* out
         [&]
         {
             const auto s = as_stream(stream);
-            AsyncScratch scratch(8, s);
-            auto* error = static_cast<uint32_t*>(scratch.pointer);
-            check_hip(hipMemsetAsync(error, 0, 8, s), "hipMemsetAsync");
-            softmax_rows(x, rows, width, out, error, s);
-            uint32_t flags[2];
-            check_hip(hipMemcpyAsync(flags, error, 8, hipMemcpyDeviceToHost, s), "read error words");
-            check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-            require(!flags[0], "softmax input must be finite");
+            ErrorWords errors(s);
+            softmax_rows(x, rows, width, out, errors.device(), s);
+            errors.check("softmax input must be finite");
         });
 }
 

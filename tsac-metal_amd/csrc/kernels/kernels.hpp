@@ -121,6 +121,11 @@ std::size_t small_gemm_max_rows();
 // K <= 2048; up to 1024 rows when the GEMM would leave most units idle).
 bool small_gemm_chosen(std::size_t M, std::size_t N, std::size_t K);
 
+// quantize_rows + linear in one launch, where the path leads to the GEMV and x and y
+// do not overlap; false (and nothing launched) where they take the two.
+bool quantizing_linear(const DeviceLinear& w, const uint16_t* x, std::size_t M, uint16_t* y, LinearPath path,
+                       uint32_t* error, hipStream_t stream);
+
 // x [M][K] BF16 -> y [M][N] like quantize_rows + linear, with the BF8L buffer in
 // a fixed per-device array (static_linear.hip) instead of caller or allocator
 // memory; padded rows x K must not exceed static_linear_max_bytes(). Fails if
