@@ -411,8 +411,10 @@ void tsac_hip_linear_destroy(tsac_hip_device_linear* linear);
 #define TSAC_HIP_PATH_SMALL 4
 
 /* PackedLinear::apply_into (src/common/packed_linear.tpp:264-302) on device
- * memory: x [M][K] BF16 -> y [M][N] BF16. quantisation scratch comes from the
- * stream-ordered allocator on `stream`. */
+ * memory: x [M][K] BF16 -> y [M][N] BF16 (M <= 8 in one launch unless y overlaps
+ * x). Waits for `stream` to report a nonfinite activation. Quantisation scratch is
+ * kept by the library between calls, at most 512 MiB a device, until the last
+ * projection is destroyed. */
 int tsac_hip_linear_apply(const tsac_hip_device_linear* linear, const uint16_t* x, size_t M,
                           uint16_t* y, int path, void* stream);
 

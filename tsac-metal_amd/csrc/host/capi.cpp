@@ -136,6 +136,24 @@ struct AsyncScratch
     }
 };
 
+// Lets this thread allocate while another one captures a graph: nothing it
+// allocates or launches here is part of that graph.
+class BesideCaptures
+{
+  public:
+    BesideCaptures()
+    {
+        (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    ~BesideCaptures()
+    {
+        (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+
+  private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // Device buffers for the projections' quantised activations, kept between calls: a
 // call waits for its stream before it returns, so a buffer given back is idle and
 // serves any stream and thread. (hipMallocAsync's pool maps its memory again after each
@@ -171,6 +189,7 @@ class ProjectionBuffers
                 return b;
             }
         }
+        const BesideCaptures relaxed;
         b.bytes = (bytes + 0xffff) / 0x10000 * 0x10000;
         check_hip(hipMalloc(&b.pointer, b.bytes), "hipMalloc");
         return b;
@@ -195,6 +214,7 @@ class ProjectionBuffers
                 unused.erase(unused.begin());
             }
         }
+        const BesideCaptures relaxed;
         for (void* p : freed)
         {
             (void)hipFree(p);
@@ -222,6 +242,7 @@ class ProjectionBuffers
                 unused_.clear();
             }
         }
+        const BesideCaptures relaxed;
         for (void* p : freed)
         {
             (void)hipFree(p);
@@ -252,6 +273,7 @@ class ErrorWords
         auto& words = unused();
         if (words.empty())
         {
+            const BesideCaptures relaxed;
             void* block = nullptr;
             check_hip(hipHostMalloc(&block, 64 * 64, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
             words.reserve(words.capacity() + 64);
