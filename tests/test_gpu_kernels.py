@@ -608,3 +608,58 @@ def test_qlinear_quantises_in_the_gemv(torch, native, oracle, k, columns):
         linear.apply(dev(torch, bad), y)
     linear.apply(dx, dx)
     assert np.array_equal(host(dx), expected)
+
+
+@pytest.mark.parametrize("count", [1, 7, 8, 9, 2047, 2048, 2055, 65536 + 3])
+def test_gelu_vectors_and_remainders(torch, native, oracle, count):
+    x = np.random.default_rng(count).integers(0, 65536, count).astype(np.uint16)
+    out = empty(torch, (count + 8,), torch.int16)
+    out.fill_(77)
+    native.gelu(dev(torch, x), out[:count])
+    assert np.array_equal(host(out)[:count], oracle.gelu_batch(x))
+    assert (host(out)[count:] == 77).all()
+
+
+@pytest.mark.parametrize("rows,width,period", [(1, 8, 1), (5, 24, 3), (7, 20, 2), (4, 512, 4), (3, 512, 100), (9, 1, 2),
+                                               (257, 1024, 12)])
+def test_add_vectors_and_periods(torch, native, rows, width, period):
+    """Rows of whole vectors or not, the second operand's rows repeating or not."""
+    rng = np.random.default_rng(rows * width)
+    a = bf16_bits(rng.standard_normal((rows, width)).astype(np.float32))
+    b = bf16_bits(rng.standard_normal((period, width)).astype(np.float32))
+    out = empty(torch, (rows, width), torch.int16)
+    native.add(dev(torch, a), dev(torch, b), rows, width, period, out)
+    assert np.array_equal(host(out), bf16_bits(bf16_float(a) + bf16_float(b[np.arange(rows) % period])))
+
+
+@pytest.mark.parametrize("width", [256, 512, 1024, 2048])
+def test_layer_norm_of_many_rows(torch, native, oracle, width):
+    """A row per wave from 2,048 rows on (on 256 compute units): the same rows give the
+    bits of a call of few rows, which spreads them."""
+    rng = np.random.default_rng(width)
+    rows = 2049
+    x = bf16_bits(rng.standard_normal((rows, width)).astype(np.float32))
+    x[::7] = bf16_bits((rng.standard_normal((len(x[::7]), width)) * 1e-19).astype(np.float32))
+    gain, bias = (dev(torch, bf16_bits(rng.standard_normal(width).astype(np.float32))) for _ in range(2))
+    many, few = (empty(torch, (rows, width), torch.int16) for _ in range(2))
+    native.layer_norm(dev(torch, x), rows, width, gain, bias, many)
+    for r in range(0, rows, 683):
+        native.layer_norm(dev(torch, x[r:r + 683]), min(683, rows - r), width, gain, bias, few[r:r + 683])
+    assert np.array_equal(host(many), host(few))
+
+
+@pytest.mark.parametrize("k", [256, 512, 1024, 2048, 4096])
+@pytest.mark.parametrize("rows", [1, 5, 33, 130])
+def test_quantised_tiles_of_wide_rows(torch, native, oracle, k, rows):
+    """Rows of 2048 and 4096 values in operand tiles, 8 rows a wave, against the row-major call."""
+    rng = np.random.default_rng(k + rows)
+    x = dev(torch, bf16_bits(rng.standard_normal((rows, k)).astype(np.float32)))
+    padded = native.tile_rows(rows)
+    q, s = empty(torch, (rows, k), torch.int8), empty(torch, (rows, k // 256), torch.float32)
+    tq, ts = empty(torch, (padded * k,), torch.int8), empty(torch, (k // 256, padded), torch.float32)
+    native.bf8l(x, rows, k, q, s)
+    native.bf8l_tiles(x, rows, k, tq, ts)
+    m, j = np.arange(rows)[:, None], np.arange(k)[None, :]
+    at = ((m // 32) * (k // 32) + j // 32) * 1024 + ((m % 32) + 32 * ((j // 16) % 2)) * 16 + j % 16
+    assert np.array_equal(tq.cpu().numpy()[at], q.cpu().numpy())
+    assert np.array_equal(ts.cpu().numpy()[:, :rows].T, s.cpu().numpy())

@@ -85,7 +85,7 @@ __device__ __forceinline__ float original_exp(float z)
     return __uint_as_float(__float_as_uint(plus_one) + (uint32_t(n) << 23));
 }
 
-// original_exp for z in [-87, 87], where its clamps and its check of the exponent
+// original_exp for z in [-88, 87], where its clamps and its check of the exponent
 // leave z and n as they are.
 __device__ __forceinline__ float exp_within(float z)
 {
@@ -113,9 +113,17 @@ __device__ __forceinline__ uint16_t gelu_bf16(uint16_t bits)
     z = z * x;
     const float half = x * 0.5f;
     z = z * -2.0f;
-    const float e = original_exp(z);
+    // original_exp between its clamps (a NaN input makes the result NaN either way).
+    const float e = exp_within(__builtin_amdgcn_fmed3f(z, -88.0f, 87.0f));
     const float denominator = e + 1.0f;
-    const float sigmoid = 2.0f / denominator;
+    // 2 / denominator, from the reciprocal's Newton step and the quotient's exact
+    // remainder: 6 instructions for the 10 of a division that also scales. The
+    // denominator lies in [1, 2^126), and there are only 65,536 inputs: every result
+    // equals the division's.
+    float inverse = __builtin_amdgcn_rcpf(denominator);
+    inverse = __builtin_fmaf(__builtin_fmaf(-denominator, inverse, 1.0f), inverse, inverse);
+    const float quotient = inverse + inverse;
+    const float sigmoid = __builtin_fmaf(__builtin_fmaf(-denominator, quotient, 2.0f), inverse, quotient);
     const float t = sigmoid - 1.0f;
     const float plus = t + 1.0f;
     return float_to_bf16(half * plus);
