@@ -587,6 +587,54 @@ def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, ki
             assert not np.isfinite(bf16_float(got[start + t][~finite])).any()
 
 
+@pytest.mark.parametrize("heads,hw", [(8, 64), (4, 128)])
+@pytest.mark.parametrize("lengths,pairs", [([64, 33, 17, 8], 32), ([64, 33, 17, 49], 1280), ([330], 8), ([129, 96], 16),
+                                           ([65, 128], 1024), ([129, 70, 100], 480), ([129, 70, 100], 96),
+                                           ([330, 257], 32)])
+@pytest.mark.parametrize("kind", ["normal", "spread", "zeros", "dead infinity"])
+def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, pairs, kind):
+    """Every choice of waves and queries a workgroup, by the count of (sequence, head)
+    pairs: the same sequences again and again equal the first ones, which equal the
+    oracle; rotated in the kernel, they equal a launch of one set."""
+    rng = np.random.default_rng(sum(lengths) + hw)
+    w, rows, sets = heads * hw, sum(lengths), max(1, pairs // (heads * len(lengths)))
+    qkv = rng.standard_normal((rows, 3 * w)).astype(np.float32)
+    if kind == "spread":
+        qkv[:, :w] *= 60
+    elif kind == "zeros":
+        qkv[:, 2 * w:2 * w + hw] = 0
+        qkv[::3, 2 * w + hw:] *= -0.0
+    elif kind == "dead infinity":
+        qkv[lengths[0] - 2, 2 * w:] = np.inf
+    qkv = bf16_bits(qkv)
+    angles = rng.standard_normal((max(lengths), hw // 2))
+    rotations = bf16_bits(np.stack([np.cos(angles), np.sin(angles)], axis=-1).reshape(-1, hw).astype(np.float32))
+    scale = np.float32(1 / np.sqrt(hw))
+
+    def run(n, rotated):
+        many = np.array(lengths * n, np.int32)
+        starts = np.cumsum(np.concatenate([[0], many[:-1]])).astype(np.int32)
+        out = empty(torch, (rows * n, w), torch.int16)
+        native.attention_causal(dev(torch, np.tile(qkv, (n, 1))), heads, hw, dev(torch, starts), dev(torch, many),
+                                dev(torch, np.zeros(len(many), np.int32)), len(many), max(lengths),
+                                dev(torch, rotations) if rotated else None, scale, out)
+        return host(out).reshape(n, rows, w)
+
+    assert np.array_equal(run(sets, True), np.tile(run(1, True), (sets, 1, 1)))
+    got = run(sets, False)
+    assert np.array_equal(got, np.tile(got[:1], (sets, 1, 1)))
+    start = 0
+    for length in lengths:
+        seq = qkv[start:start + length]
+        q, k, v = seq[:, :w].copy(), seq[:, w:2 * w].copy(), seq[:, 2 * w:].copy()
+        for t in range(length):
+            expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, False)
+            finite = np.isfinite(bf16_float(expected))
+            assert np.array_equal(got[0, start + t][finite], expected[finite]), (length, t)
+            assert not np.isfinite(bf16_float(got[0, start + t][~finite])).any()
+        start += length
+
+
 @pytest.mark.parametrize("k", [256, 512, 1024, 2048, 4096])
 @pytest.mark.parametrize("columns", range(1, 9))
 def test_qlinear_quantises_in_the_gemv(torch, native, oracle, k, columns):

@@ -10,7 +10,7 @@
 // Decode (one query per sequence): each (sequence, head)'s 64-key blocks are
 // spread over several workgroups of one launch, one wave per block; the last
 // workgroup to arrive merges the block records in ascending order.
-// Prefill (encode, all queries known): one workgroup per (sequence, head, 32-query
+// Prefill (encode, all queries known): one workgroup per (sequence, head, query
 // tile), one wave per causal key block, the blocks' sums merged in ascending order.
 #include "attention.hpp"
 #include "device_numeric.hpp"
@@ -422,8 +422,7 @@ __global__ __launch_bounds__(decode_waves * 64) void decode_attention_kernel(
 
 // ------------------------------------------------------------------ prefill
 
-constexpr int tile = 64;                          // keys of a block
-constexpr int per_lane = 4, queries = 8 * per_lane; // of a wave
+constexpr int tile = 64; // keys of a block
 
 // 16 bytes at any 2-byte-aligned address.
 __device__ __forceinline__ u32x4 load16(const uint16_t* from)
@@ -467,14 +466,15 @@ __device__ __forceinline__ void tile_fence()
 }
 
 // LDS of a workgroup of W waves: the query tile, each wave's key (32
-// coordinates of 64 keys at a time), weight (16 keys x 32 queries, in the keys'
+// coordinates of 64 keys at a time), weight (16 keys x the queries, in the keys'
 // place) and value tiles (16 keys x 64 coordinates), and the merged state that
 // the waves hand on block by block. Rows are padded so that eight lanes reading or
 // writing 16 bytes of eight rows meet eight different 16-byte banks.
 constexpr int phase_coordinates = 32, chunk_keys = 16, value_coordinates = 64;
 
-template <int HW, int W> struct PrefillShared
+template <int HW, int W, int queries> struct PrefillShared
 {
+    static constexpr int per_lane = queries / 8;
     static constexpr int q_row = HW + 8, k_row = phase_coordinates + 8, p_row = queries + 4;
     union Wave
     {
@@ -492,7 +492,7 @@ template <int HW, int W> struct PrefillShared
     int turn[HW / value_coordinates];
 };
 
-// A workgroup takes 32 queries of one (sequence, head); its W waves take the
+// A workgroup takes 8, 16 or 32 queries of one (sequence, head); its W waves take the
 // causal 64-key blocks in turn, each whole: lane (lq, lk) = (lane / 8, lane % 8)
 // holds queries lq + 8 a and, for scores, keys lk + 8 b, so that the 8-lane
 // butterfly on each register followed by the register pair tree is exactly the
@@ -510,14 +510,24 @@ template <int HW, int W> struct PrefillShared
 // with 4 x 4 sums a thread (before) was bound by its LDS reads and barriers. Four
 // waves per SIMD (128 registers) spill and gain nothing. Measured on 3 sequences of
 // 861 rows, before and now: 16 heads of 64 244 -> 136 us, 4 heads of 128 287 -> 88 us;
-// of 100 rows 25.5 -> 21.6 and 38 -> 34 us; of 2,580 rows 1,222 -> 910 and 942 -> 494.
-template <int HW, int W, bool Rotary>
+// of 2,580 rows 1,222 -> 910 and 942 -> 494. 8 and 16 queries (the launch says when)
+// shorten a block's chain: 4 sequences of 64 rows 15 -> 9.4 and 23 -> 16 us (32 queries:
+// 19 and 34), 4 of 120 rows 27 -> 18 and 41 -> 16.
+template <int HW, int W, int queries, bool Rotary>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) void prefill_kernel(
     const uint16_t* __restrict__ qkv, int width, const int* __restrict__ sequence_start,
     const int* __restrict__ sequence_length, const int* __restrict__ sequence_replay,
     const uint16_t* __restrict__ rotations, int heads, float scale, uint16_t* __restrict__ out)
 {
-    using Shared = PrefillShared<HW, W>;
+    using Shared = PrefillShared<HW, W, queries>;
+    constexpr int per_lane = Shared::per_lane;
+    using Weights = float __attribute__((ext_vector_type(per_lane)));
+    // With one query a lane, registers hold a block's keys and a half's values, so that
+    // their loads wait for memory once.
+    constexpr bool ahead = per_lane == 1;
+    constexpr int phases = HW / phase_coordinates, held_phases = ahead ? phases : 1;
+    constexpr int chunks = tile / chunk_keys, held_chunks = ahead ? chunks : 1;
+    constexpr int score_steps = ahead ? 2 : 1, key_steps = ahead ? 8 : 2; // unrolled
     constexpr int q_row = Shared::q_row, k_row = Shared::k_row, p_row = Shared::p_row;
     __shared__ Shared shared;
     const int sequence = blockIdx.x / heads, head = blockIdx.x % heads;
@@ -570,7 +580,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
     {
         const int k0 = block * tile;
         // Keys past the sequence read its last one, and are masked out.
-        u32x4 held[4], held_rotation[4] = {};
+        u32x4 held[held_phases][4], held_rotation[held_phases][4] = {};
         const auto fetch_keys = [&](int phase)
         {
 #pragma unroll
@@ -578,11 +588,34 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
             {
                 const int i = lane + 64 * j, r = i / 4, c = phase * phase_coordinates + i % 4 * 8;
                 const int position = k0 + r < length ? k0 + r : length - 1;
-                held[j] = *reinterpret_cast<const u32x4*>(base + std::size_t(position) * stride + width + c);
+                held[phase % held_phases][j] =
+                    *reinterpret_cast<const u32x4*>(base + std::size_t(position) * stride + width + c);
                 if constexpr (Rotary)
                 {
-                    held_rotation[j] = load16(rotations + std::size_t(position) * HW + c);
+                    held_rotation[phase % held_phases][j] = load16(rotations + std::size_t(position) * HW + c);
                 }
+            }
+        };
+        // Value rows, 16 keys x 64 coordinates at a time: rows past the sequence
+        // read its last one, and their weights are never applied.
+        u32x4 held_values[held_chunks][2];
+        const auto fetch_values = [&](int half, int chunk)
+        {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+            {
+                const int i = lane + 64 * j, r = k0 + chunk * chunk_keys + i / 8;
+                const int position = r < length ? r : length - 1;
+                held_values[chunk % held_chunks][j] = *reinterpret_cast<const u32x4*>(
+                    base + std::size_t(position) * stride + 2 * width + half * value_coordinates + i % 8 * 8);
+            }
+        };
+        const auto fetch_first_values = [&](int half)
+        {
+#pragma unroll
+            for (int chunk = 0; chunk < held_chunks; ++chunk)
+            {
+                fetch_values(half, chunk);
             }
         };
         float dot[per_lane][8]; // scores, then weights
@@ -595,19 +628,19 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
                 dot[a][b] = 0.0f;
             }
         }
-        for (int phase = 0; phase < HW / phase_coordinates; ++phase)
+        const auto score_phase = [&](int phase)
         {
-            fetch_keys(phase);
             tile_fence();
 #pragma unroll
             for (int j = 0; j < 4; ++j)
             {
                 const int i = lane + 64 * j, r = i / 4, c = i % 4;
                 *reinterpret_cast<u32x4*>(mine.k + r * k_row + c * 8) =
-                    Rotary ? rotate8(held[j], held_rotation[j]) : held[j];
+                    Rotary ? rotate8(held[phase % held_phases][j], held_rotation[phase % held_phases][j])
+                           : held[phase % held_phases][j];
             }
             tile_fence();
-#pragma unroll 1
+#pragma unroll score_steps
             for (int c = 0; c < phase_coordinates / 8; ++c)
             {
                 u32x4 qu[per_lane], ku[8];
@@ -647,23 +680,34 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
                     }
                 }
             }
-        }
-
-        // Value rows, 16 keys x 64 coordinates at a time: rows past the sequence
-        // read its last one, and their weights are never applied.
-        u32x4 held_values[2];
-        const auto fetch_values = [&](int half, int chunk)
+        };
+        if constexpr (ahead)
         {
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int phase = 0; phase < phases; ++phase)
             {
-                const int i = lane + 64 * j, r = k0 + chunk * chunk_keys + i / 8;
-                const int position = r < length ? r : length - 1;
-                held_values[j] = *reinterpret_cast<const u32x4*>(base + std::size_t(position) * stride + 2 * width +
-                                                                 half * value_coordinates + i % 8 * 8);
+                fetch_keys(phase);
             }
-        };
-        fetch_values(0, 0);
+            fetch_first_values(0);
+#pragma unroll
+            for (int phase = 0; phase < phases; ++phase)
+            {
+                score_phase(phase);
+            }
+        }
+        else
+        {
+            for (int phase = 0; phase < phases; ++phase)
+            {
+                fetch_keys(phase);
+                score_phase(phase);
+            }
+        }
+
+        if constexpr (!ahead)
+        {
+            fetch_first_values(0);
+        }
 
         // A query's last live key of the block (all of them but for the last block's).
         int last_key[per_lane];
@@ -780,10 +824,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
                 }
                 if (Careful || half > 0)
                 {
-                    fetch_values(half, 0);
+                    fetch_first_values(half);
                 }
 #pragma unroll
-                for (int chunk = 0; chunk < tile / chunk_keys; ++chunk)
+                for (int chunk = 0; chunk < chunks; ++chunk)
                 {
                     if (chunk * chunk_keys > last_live)
                     {
@@ -794,18 +838,23 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
                     for (int i = 0; i < 2; ++i)
                     {
                         const int b = chunk * 2 + i;
-                        *reinterpret_cast<f32x4*>(mine.p + (lk + 8 * i) * p_row + lq * 4) =
-                            f32x4{dot[0][b], dot[1][b], dot[2][b], dot[3][b]};
-                        *reinterpret_cast<u32x4*>(mine.v + (lane + 64 * i) * 8) = held_values[i];
+                        Weights w;
+#pragma unroll
+                        for (int a = 0; a < per_lane; ++a)
+                        {
+                            w[a] = dot[a][b];
+                        }
+                        *reinterpret_cast<Weights*>(mine.p + (lk + 8 * i) * p_row + lq * per_lane) = w;
+                        *reinterpret_cast<u32x4*>(mine.v + (lane + 64 * i) * 8) = held_values[chunk % held_chunks][i];
                     }
                     tile_fence();
-                    if (chunk + 1 < tile / chunk_keys)
+                    if (!ahead && chunk + 1 < chunks)
                     {
                         fetch_values(half, chunk + 1);
                     }
                     const auto term = [&](int t)
                     {
-                        const f32x4 w = *reinterpret_cast<const f32x4*>(mine.p + t * p_row + lq * 4);
+                        const Weights w = *reinterpret_cast<const Weights*>(mine.p + t * p_row + lq * per_lane);
                         float value[8];
                         widen8(*reinterpret_cast<const u32x4*>(mine.v + t * value_coordinates + lk * 8), value);
 #pragma unroll
@@ -829,7 +878,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
                     }
                     else
                     {
-#pragma unroll 2
+#pragma unroll key_steps
                         for (int t = 0; t < chunk_keys; ++t)
                         {
                             term(t);
@@ -1229,29 +1278,64 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
         check_hip(hipGetLastError(), "attention prefill launch");
         return;
     }
-    const dim3 grid(unsigned(sequences * heads), unsigned((max_length + queries - 1) / queries));
-    const auto launch = [&](auto rotary, auto plain, int waves)
+    // Waves and queries of a workgroup, by the blocks of the longest history and by how
+    // many workgroups there are for the device's units (256). Small query tiles shorten
+    // the chain of a block (8 queries: a quarter of the sums a lane, and its loads wait
+    // for memory once), which is the time of a launch that leaves units idle; large ones
+    // read and rotate a key for more queries; more waves take more blocks at a time, and
+    // are idle slots where there are none. us, waves x queries, 16 heads of 64 | 4 of 128:
+    //   rows x sequences       1x8   4x8   8x8  1x16  2x16  4x32 |  1x8   4x8   8x8  1x16  2x16  4x32 (8x32 from 300 x 2 on)
+    //   64 x 4                 9.5   9.5    15  13.9  13.3  19.2 | 15.7  15.5  15.5  24.0  23.3  33.5
+    //   64 x 64                 38    52   220    28    32    40 |   21    32    98    26    24    35
+    //   64 x 1000              580   827  3763   369   406   591 |  263   364  1629   193   223   352
+    //   120 x 4                 17    18    31    25    16    21 |   28    16    16    43    24    35
+    //   120 x 100              152   292   735   105   116   203 |   74   133   325    69    64   111
+    //   300 x 2                 37    29    43    57    34    38 |   65    29    29   101    63    38
+    //   430 x 1                 50    27    37    78    45    27 |   91    30    21   141    83    44
+    //   430 x 20               277   402   648   176   185   258 |  146   184   277   146   108   131
+    //   862 x 3                161   194   257   154   115   120 |  183    94   123   286   146    82
+    //   2580 x 1               457   473   551   445   321   297 |  529   235   260   826   423   205
+    const std::size_t units = std::size_t(compute_units());
+    constexpr std::integral_constant<int, 1> one;
+    constexpr std::integral_constant<int, 2> two;
+    constexpr std::integral_constant<int, 4> four;
+    constexpr std::integral_constant<int, 8> eight;
+    constexpr std::integral_constant<int, 16> sixteen;
+    constexpr std::integral_constant<int, 32> thirty_two;
+    const auto tiles = [&](std::size_t queries) { return sequences * heads * ((max_length + queries - 1) / queries); };
+    const auto launch = [&](auto rotary, auto plain, int waves, std::size_t queries)
     {
-        (rotations ? rotary : plain)<<<grid, 64 * waves, 0, stream>>>(qkv, int(width), sequence_start, sequence_length, sequence_replay,
-                                                rotations, int(heads), scale, out);
+        const dim3 grid(unsigned(sequences * heads), unsigned((max_length + queries - 1) / queries));
+        (rotations ? rotary : plain)<<<grid, 64 * waves, 0, stream>>>(
+            qkv, int(width), sequence_start, sequence_length, sequence_replay, rotations, int(heads), scale, out);
     };
-    // Eight waves take twice the blocks of a query tile at a time, which pays only
-    // where histories have more than four blocks and the grid alone does not fill the
-    // device (16 heads of 64, 4 against 8 waves: one sequence of 862 rows, 432
-    // workgroups, 75 and 63 us; three of 430, 672 workgroups, 53 and 70 us; 4 heads of
-    // 128, three of 861, 324 workgroups, 133 and 88 us).
-    const bool eight =
-        max_length > 4 * tile && std::size_t(grid.x) * grid.y < 2 * std::size_t(compute_units());
-    if (head_width == 64)
+    const auto by_width = [&](auto head)
     {
-        eight ? launch(prefill_kernel<64, 8, true>, prefill_kernel<64, 8, false>, 8)
-              : launch(prefill_kernel<64, 4, true>, prefill_kernel<64, 4, false>, 4);
-    }
-    else
-    {
-        eight ? launch(prefill_kernel<128, 8, true>, prefill_kernel<128, 8, false>, 8)
-              : launch(prefill_kernel<128, 4, true>, prefill_kernel<128, 4, false>, 4);
-    }
+        constexpr int HW = decltype(head)::value;
+        const auto variant = [&](auto waves, auto queries)
+        {
+            constexpr int W = decltype(waves)::value, Q = decltype(queries)::value;
+            launch(prefill_kernel<HW, W, Q, true>, prefill_kernel<HW, W, Q, false>, W, Q);
+        };
+        if (max_length <= tile)
+        {
+            tiles(8) <= 8 * units ? variant(one, eight) : variant(one, sixteen);
+        }
+        else if (tiles(8) <= 4 * units)
+        {
+            tiles(8) <= 2 * units && max_length > 4 * tile ? variant(eight, eight) : variant(four, eight);
+        }
+        else if (max_length <= 2 * tile || tiles(16) >= 12 * units ||
+                 (tiles(16) >= 8 * units && max_length <= 8 * tile))
+        {
+            variant(two, sixteen);
+        }
+        else
+        {
+            max_length > 4 * tile && tiles(32) < 2 * units ? variant(eight, thirty_two) : variant(four, thirty_two);
+        }
+    };
+    head_width == 64 ? by_width(std::integral_constant<int, 64>{}) : by_width(std::integral_constant<int, 128>{});
     check_hip(hipGetLastError(), "attention prefill launch");
 }
 } // namespace tsac_hip
