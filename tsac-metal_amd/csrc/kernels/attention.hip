@@ -510,7 +510,7 @@ template <int HW, int W, int queries> struct PrefillShared
 // with 4 x 4 sums a thread (before) was bound by its LDS reads and barriers. Four
 // waves per SIMD (128 registers) spill and gain nothing. Measured on 3 sequences of
 // 861 rows, before and now: 16 heads of 64 244 -> 136 us, 4 heads of 128 287 -> 88 us;
-// of 2,580 rows 1,222 -> 910 and 942 -> 494. 8 and 16 queries (the launch says when)
+// of 2,580 rows 1,222 -> 910 (819 unrotated, with 16 queries) and 942 -> 494. 8 and 16 queries (the launch says when)
 // shorten a block's chain: 4 sequences of 64 rows 15 -> 9.4 and 23 -> 16 us (32 queries:
 // 19 and 34), 4 of 120 rows 27 -> 18 and 41 -> 16.
 template <int HW, int W, int queries, bool Rotary>
