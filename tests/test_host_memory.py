@@ -1,0 +1,66 @@
+"""The library's memory management and launch shapes on the CPU: a child process loads
+tests/support/host_hip.cpp, which makes the HIP calls on the host alone, before
+libtsac_hip.so, and goes through the C ABI as a program does."""
+import pathlib
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+TESTS = pathlib.Path(__file__).resolve().parent
+
+PRELUDE = """
+import ctypes, sys
+sys.path.insert(0, {package!r})
+hip = ctypes.CDLL({hip!r}, mode=ctypes.RTLD_GLOBAL)
+hip.host_hip_total.argtypes = [ctypes.c_size_t]
+hip.host_hip_used.restype = ctypes.c_size_t
+hip.host_hip_count.argtypes, hip.host_hip_count.restype = [ctypes.c_char_p], ctypes.c_long
+hip.host_hip_launches.restype = ctypes.c_char_p
+import numpy as np
+from tsac_hip import native, synthetic
+lib = native.library()
+GiB, MiB = 1 << 30, 1 << 20
+
+def counts():
+    return {{name: hip.host_hip_count(name.encode()) for name in ("hipMalloc", "hipFree", "hipMallocAsync", "hipFreeAsync")}}
+
+def launches():
+    return [line.split() for line in hip.host_hip_launches().decode().splitlines()]
+"""
+
+
+@pytest.fixture(scope="session")
+def host_hip(tmp_path_factory):
+    target = tmp_path_factory.mktemp("host_hip") / "libhost_hip.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    str(TESTS / "support" / "host_hip.cpp"), "-o", str(target)], check=True)
+    return target
+
+
+def run(host_hip, body):
+    program = PRELUDE.format(package=str(TESTS.parent / "tsac-metal_amd"), hip=str(host_hip)) + textwrap.dedent(body)
+    result = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, timeout=300)
+    assert result.returncode == 0, f"status {result.returncode}\n{result.stdout}{result.stderr[-3000:]}"
+    return result.stdout
+
+
+def test_encode_without_page_locked_memory(host_hip):
+    """Where page-locked memory cannot grow, an encode goes through pageable memory, and
+    the session's later ones, small or large, are as good as before."""
+    run(host_hip, """
+    geometry = synthetic.Geometry(width=256, heads=2, head_width=128, ffn=512, temporal_layers=1, codebook_layers=1,
+                                  latent=256)
+    session = native.HipModel(synthetic.random_model(geometry, seed=1)).session()
+    def encode(frames):
+        tokens = synthetic.pattern_tokens(frames * 12)
+        return session.encode(native.header(frames, 1, 1, 12), tokens)
+    small, large = encode(8), native.HipModel(synthetic.random_model(geometry, seed=1)).session()
+    want = large.encode(native.header(40, 1, 1, 12), synthetic.pattern_tokens(40 * 12))
+    hip.host_hip_pinned_fails(1)
+    assert encode(40) == want
+    assert encode(8) == small
+    hip.host_hip_pinned_fails(0)
+    assert encode(40) == want and encode(8) == small
+    """)

@@ -108,19 +108,39 @@ PinnedBuffer::~PinnedBuffer()
     }
 }
 
-void PinnedBuffer::reserve(std::size_t bytes)
+hipError_t PinnedBuffer::grow(std::size_t bytes)
 {
     if (bytes <= bytes_)
     {
-        return;
+        return hipSuccess;
+    }
+    void* grown = nullptr;
+    if (const hipError_t status = hipHostMalloc(&grown, bytes, hipHostMallocDefault); status != hipSuccess)
+    {
+        return status;
     }
     if (data_)
     {
         (void)hipHostFree(data_);
-        data_ = nullptr;
     }
-    check_hip(hipHostMalloc(&data_, bytes, hipHostMallocDefault), "hipHostMalloc");
+    data_ = grown;
     bytes_ = bytes;
+    return hipSuccess;
+}
+
+void PinnedBuffer::reserve(std::size_t bytes)
+{
+    check_hip(grow(bytes), "hipHostMalloc");
+}
+
+bool PinnedBuffer::try_reserve(std::size_t bytes)
+{
+    if (grow(bytes) == hipSuccess)
+    {
+        return true;
+    }
+    (void)hipGetLastError(); // not the next launch's error
+    return false;
 }
 
 void* Arena::get(const std::string& name, std::size_t bytes)
@@ -691,13 +711,12 @@ std::vector<uint8_t> Session::encode(Header h, const uint16_t* tokens, std::size
     require(model_->limits().file_bytes >= 19, "the stream limit is below the 19-byte FBAZ framing");
     const uint32_t crc = token_crc32(tokens, count);
     // Page-locked up to 16 MiB (some eight minutes of stereo), where the copy from the
-    // device is one transfer.
+    // device is one transfer; pageable beyond, or where page-locked memory is short.
     constexpr std::size_t staged = std::size_t(16) << 20;
     std::vector<uint16_t> unstaged;
     uint16_t* splits = nullptr;
-    if (count * 32 <= staged)
+    if (count * 32 <= staged && staging_splits_.try_reserve(std::max<std::size_t>(count, 1) * 32))
     {
-        staging_splits_.reserve(std::max<std::size_t>(count, 1) * 32);
         splits = staging_splits_.as<uint16_t>();
     }
     else

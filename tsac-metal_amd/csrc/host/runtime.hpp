@@ -75,19 +75,24 @@ private:
     std::size_t bytes_ = 0;
 };
 
-// Page-locked host staging.
+// Page-locked host staging. A buffer that cannot grow stays as it was.
 class PinnedBuffer
 {
 public:
     PinnedBuffer() = default;
     ~PinnedBuffer();
+    PinnedBuffer(const PinnedBuffer&) = delete;
+    PinnedBuffer& operator=(const PinnedBuffer&) = delete;
     void reserve(std::size_t bytes);
+    // False, with no error left behind, where page-locked memory is short.
+    bool try_reserve(std::size_t bytes);
     template <class T> T* as() const
     {
         return static_cast<T*>(data_);
     }
 
 private:
+    hipError_t grow(std::size_t bytes);
     void* data_ = nullptr;
     std::size_t bytes_ = 0;
 };
