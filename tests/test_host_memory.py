@@ -64,3 +64,16 @@ def test_encode_without_page_locked_memory(host_hip):
     hip.host_hip_pinned_fails(0)
     assert encode(40) == want and encode(8) == small
     """)
+
+
+def test_a_failed_allocation_leaves_no_error_behind(host_hip):
+    """A call that failed for want of device memory does not fail the next call's launches."""
+    run(host_hip, """
+    linear = native.DeviceLinear(np.zeros((256, 256), np.int8), np.ones((1, 256), np.float32), np.zeros(256, np.float32))
+    def apply(rows):
+        return lib.tsac_hip_linear_apply(linear.handle, 1 << 20, rows, 1 << 40, native.PATH_AUTO, None)
+    hip.host_hip_total(hip.host_hip_used())
+    assert apply(1 << 20) != 0 and b"out of memory" in lib.tsac_hip_last_error()
+    hip.host_hip_total(GiB)
+    assert apply(4) == 0, lib.tsac_hip_last_error()
+    """)

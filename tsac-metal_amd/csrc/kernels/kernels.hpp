@@ -29,6 +29,7 @@ inline void check_hip(hipError_t status, const char* what)
 {
     if (status != hipSuccess)
     {
+        (void)hipGetLastError(); // reported here, not by the next launch
         throw Error(std::string(what) + ": " + hipGetErrorString(status));
     }
 }
