@@ -412,9 +412,10 @@ void tsac_hip_linear_destroy(tsac_hip_device_linear* linear);
 
 /* PackedLinear::apply_into (src/common/packed_linear.tpp:264-302) on device
  * memory: x [M][K] BF16 -> y [M][N] BF16 (M <= 8 in one launch unless y overlaps
- * x). Waits for `stream` to report a nonfinite activation. Quantisation scratch is
+ * x). Waits for `stream` to report a nonfinite activation, so `stream` must not be
+ * captured, nor any other one in the global capture mode. Quantisation scratch is
  * kept by the library between calls, at most 512 MiB a device, until the last
- * projection is destroyed. */
+ * projection is destroyed; calls that find no room in it take stream-ordered memory. */
 int tsac_hip_linear_apply(const tsac_hip_device_linear* linear, const uint16_t* x, size_t M,
                           uint16_t* y, int path, void* stream);
 

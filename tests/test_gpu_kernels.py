@@ -711,3 +711,76 @@ def test_quantised_tiles_of_wide_rows(torch, native, oracle, k, rows):
     at = ((m // 32) * (k // 32) + j // 32) * 1024 + ((m % 32) + 32 * ((j // 16) % 2)) * 16 + j % 16
     assert np.array_equal(tq.cpu().numpy()[at], q.cpu().numpy())
     assert np.array_equal(ts.cpu().numpy()[:, :rows].T, s.cpu().numpy())
+
+
+def test_qlinear_calls_overlap_on_threads(torch, native):
+    """Calls of different sizes on threads and streams of their own share the kept buffers:
+    each gives what it gives alone."""
+    import threading
+
+    rng = np.random.default_rng(5)
+    linear = native.DeviceLinear(*random_linear(rng, 1024, 1024))
+    rows = (5, 40, 700, 5000, 30000)
+    inputs = [dev(torch, bf16_bits(rng.standard_normal((m, 1024)).astype(np.float32))) for m in rows]
+    outputs = [[empty(torch, (m, 1024), torch.int16) for _ in range(8)] for m in rows]
+    alone = [empty(torch, (m, 1024), torch.int16) for m in rows]
+    for x, y in zip(inputs, alone):
+        linear.apply(x, y)
+    torch.cuda.synchronize()
+    failures = []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            for y in outputs[i]:
+                linear.apply(inputs[i], y, stream=stream)
+        except Exception as e:  # noqa: BLE001
+            failures.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(rows))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
+    for i, m in enumerate(rows):
+        assert all(bool((y == alone[i]).all()) for y in outputs[i]), m
+
+
+def test_qlinear_buffer_grows_beside_a_capture(torch, native):
+    """One thread's call allocates its buffer while another thread's stream is captured in
+    the thread-local mode (the global one forbids the call's wait for its stream);
+    neither disturbs the other, and the graph replays like its eager calls."""
+    import threading
+
+    rng = np.random.default_rng(6)
+    linear = native.DeviceLinear(*random_linear(rng, 1024, 256))
+    x = dev(torch, bf16_bits(rng.standard_normal((150000, 1024)).astype(np.float32)))
+    y, alone = empty(torch, (150000, 256), torch.int16), empty(torch, (150000, 256), torch.int16)
+    small, wanted, captured = dev(torch, np.arange(65536, dtype=np.uint16)), *(empty(torch, (65536,), torch.int16)
+                                                                               for _ in range(2))
+    native.gelu(small, wanted)
+    stream, capturing = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    failures = []
+
+    def work():
+        try:
+            linear.apply(x, y, stream=stream)
+        except Exception as e:  # noqa: BLE001
+            failures.append(e)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=capturing, capture_error_mode="thread_local"):
+        native.gelu(small, captured)
+        thread = threading.Thread(target=work)
+        thread.start()
+        thread.join()
+    assert not failures, failures
+    linear.apply(x, alone)
+    assert bool((y == alone).all())
+    for _ in range(3):
+        captured.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((captured == wanted).all())

@@ -77,3 +77,85 @@ def test_a_failed_allocation_leaves_no_error_behind(host_hip):
     hip.host_hip_total(GiB)
     assert apply(4) == 0, lib.tsac_hip_last_error()
     """)
+
+
+PROJECTION = """
+def projection(k):
+    return native.DeviceLinear(np.zeros((256, k), np.int8), np.ones((k // 256, 256), np.float32), np.zeros(256, np.float32))
+
+def apply(linear, bytes_, ok=True):
+    # rows in operand tiles, of about that many quantised bytes
+    status = lib.tsac_hip_linear_apply(linear.handle, 1 << 44, bytes_ // linear.K, 1 << 45, native.PATH_GEMM, None)
+    assert (status == 0) == ok, lib.tsac_hip_last_error()
+
+linear = projection(4096)
+base = hip.host_hip_used()
+"""
+
+
+def test_projection_buffers_outlive_larger_calls(host_hip):
+    """Calls past the kept bytes take stream-ordered memory, as any other memory
+    allocates and frees, and leave the kept buffers alone; sizes that fit are allocated
+    once, and their frees (each waits for the device) end with the growing."""
+    run(host_hip, PROJECTION + textwrap.dedent("""
+    apply(linear, 16 * MiB)
+    kept = hip.host_hip_used()
+    assert kept - base >= 16 * MiB
+    before = counts()
+    for _ in range(5):
+        apply(linear, 600 * MiB)
+        assert hip.host_hip_used() == kept
+        apply(linear, 16 * MiB)
+    after = counts()
+    assert after["hipMalloc"] == before["hipMalloc"] and after["hipFree"] == before["hipFree"]
+    assert after["hipMallocAsync"] - before["hipMallocAsync"] == 5
+    for size in (127, 400, 300, 16, 480):  # growing past the bound takes the smaller ones' place
+        apply(linear, size * MiB)
+        assert hip.host_hip_used() - base <= 512 * MiB
+    before = counts()
+    for size in (16, 480, 127, 300, 600, 400):
+        apply(linear, size * MiB)
+    after = counts()
+    assert after["hipMalloc"] == before["hipMalloc"] and after["hipFree"] == before["hipFree"]
+    del linear
+    import gc; gc.collect()
+    assert hip.host_hip_used() == 0
+    """))
+
+
+def test_projection_buffers_give_way_where_memory_is_short(host_hip):
+    """Idle buffers that are too small are freed where a larger one, kept or
+    stream-ordered, finds no memory; a call that finds none all the same fails alone."""
+    run(host_hip, PROJECTION + textwrap.dedent("""
+    apply(linear, 100 * MiB)
+    hip.host_hip_total(base + 260 * MiB)
+    apply(linear, 200 * MiB)
+    hip.host_hip_total(base + 660 * MiB)
+    apply(linear, 600 * MiB)
+    apply(linear, 100 * MiB)
+    hip.host_hip_total(base + 300 * MiB)
+    apply(linear, 400 * MiB, ok=False)
+    apply(linear, 600 * MiB, ok=False)
+    apply(linear, 100 * MiB)
+    """))
+
+
+def test_projection_buffers_of_overlapping_calls(host_hip):
+    run(host_hip, PROJECTION + textwrap.dedent("""
+    import random, threading
+    failures = []
+    def work(seed):
+        rng = random.Random(seed)
+        for _ in range(200):
+            size = rng.choice((1, 20, 130, 300, 510, 700)) * MiB
+            if lib.tsac_hip_linear_apply(linear.handle, 1 << 44, size // 4096, 1 << 45, native.PATH_GEMM, None):
+                failures.append(lib.tsac_hip_last_error())
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for t in threads: t.start()
+    for t in threads: t.join()
+    assert not failures, failures
+    assert hip.host_hip_used() - base <= 512 * MiB
+    del linear
+    import gc; gc.collect()
+    assert hip.host_hip_used() == 0
+    """))

@@ -12,6 +12,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <optional>
 #include <utility>
 
 using namespace tsac_hip;
@@ -136,8 +137,9 @@ struct AsyncScratch
     }
 };
 
-// Lets this thread allocate while another one captures a graph: nothing it
-// allocates or launches here is part of that graph.
+// Lets this thread allocate while a graph is captured from another stream: nothing it
+// allocates or launches here is part of that graph. (A capture in the global mode
+// forbids the calls' wait for their stream on every thread, and is ended by it.)
 class BesideCaptures
 {
   public:
@@ -158,67 +160,99 @@ class BesideCaptures
 // call waits for its stream before it returns, so a buffer given back is idle and
 // serves any stream and thread. (hipMallocAsync's pool maps its memory again after each
 // synchronisation, a release threshold or not: a 30,960-row block spent 300 us between
-// two kernels on it.) At most `kept` bytes a device stay; the last projection
-// destroyed frees them.
+// two kernels on it.) The buffers of a device, in use or not, come to at most `kept`
+// bytes, and the last projection destroyed frees them. Memory is freed (which waits for
+// the whole device) only where a buffer has to grow, and never once a program's sizes
+// have been seen: a call that finds no room takes stream-ordered memory instead.
 class ProjectionBuffers
 {
+    using Buffers = std::multimap<std::size_t, void*>; // by size
+
   public:
     static constexpr std::size_t kept = std::size_t(512) << 20;
 
     struct Buffer
     {
-        void* pointer = nullptr;
-        std::size_t bytes = 0;
+        Buffers::node_type node; // given back without an allocation
         int device = 0;
+        void* pointer() const
+        {
+            return node.empty() ? nullptr : node.mapped();
+        }
     };
 
-    // The smallest unused buffer of at least `bytes`, or a new one.
+    // The smallest unused buffer of at least `bytes`, or a new one in the place of
+    // unused ones that are too small; none where the kept bytes leave no room.
     Buffer take(std::size_t bytes)
     {
         Buffer b;
         check_hip(hipGetDevice(&b.device), "hipGetDevice");
+        bytes = (bytes + 0xffff) / 0x10000 * 0x10000;
+        Buffers made, freed;
         {
             const std::lock_guard<std::mutex> lock(mutex_);
-            auto& unused = unused_[b.device];
-            auto found = unused.lower_bound(bytes);
-            if (found != unused.end())
+            Pool& pool = pools_[b.device];
+            if (const auto found = pool.unused.lower_bound(bytes); found != pool.unused.end())
             {
-                b.bytes = found->first;
-                b.pointer = found->second;
-                unused.erase(found);
+                b.node = pool.unused.extract(found);
                 return b;
             }
+            std::size_t idle = 0;
+            for (const auto& [size, pointer] : pool.unused)
+            {
+                idle += size;
+            }
+            if (pool.total - idle + bytes > kept)
+            {
+                return b;
+            }
+            made.emplace(bytes, nullptr);
+            while (pool.total + bytes > kept)
+            {
+                pool.drop(std::prev(pool.unused.end()), freed);
+            }
+            pool.total += bytes;
         }
-        const BesideCaptures relaxed;
-        b.bytes = (bytes + 0xffff) / 0x10000 * 0x10000;
-        check_hip(hipMalloc(&b.pointer, b.bytes), "hipMalloc");
-        return b;
-    }
-    // Keeps an idle buffer, freeing the smallest ones beyond the bound.
-    void give(const Buffer& b)
-    {
-        std::vector<void*> freed;
+        release(freed);
+        b.node = made.extract(made.begin());
+        hipError_t status = allocate(&b.node.mapped(), bytes);
+        if (status != hipSuccess)
+        {
+            release_unused(b.device);
+            status = allocate(&b.node.mapped(), bytes);
+        }
+        if (status != hipSuccess)
         {
             const std::lock_guard<std::mutex> lock(mutex_);
-            auto& unused = unused_[b.device];
-            unused.emplace(b.bytes, b.pointer);
-            std::size_t total = 0;
-            for (const auto& [bytes, pointer] : unused)
-            {
-                total += bytes;
-            }
-            while (total > kept || (!projections_ && !unused.empty()))
-            {
-                total -= unused.begin()->first;
-                freed.push_back(unused.begin()->second);
-                unused.erase(unused.begin());
-            }
+            pools_[b.device].total -= bytes;
+            check_hip(status, "hipMalloc");
         }
-        const BesideCaptures relaxed;
-        for (void* p : freed)
+        return b;
+    }
+    // Keeps an idle buffer.
+    void give(Buffer& b)
+    {
+        Buffers freed;
         {
-            (void)hipFree(p);
+            const std::lock_guard<std::mutex> lock(mutex_);
+            Pool& pool = pools_[b.device];
+            const auto at = pool.unused.insert(std::move(b.node));
+            if (!projections_)
+            {
+                pool.drop(at, freed);
+            }
         }
+        release(freed);
+    }
+    // Frees a device's unused buffers.
+    void release_unused(int device)
+    {
+        Buffers freed;
+        {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            pools_[device].drop_all(freed);
+        }
+        release(freed);
     }
     void created()
     {
@@ -227,31 +261,65 @@ class ProjectionBuffers
     }
     void destroyed()
     {
-        std::vector<void*> freed;
+        Buffers freed;
         {
             const std::lock_guard<std::mutex> lock(mutex_);
             if (--projections_ == 0)
             {
-                for (auto& [device, unused] : unused_)
+                for (auto& [device, pool] : pools_)
                 {
-                    for (const auto& [bytes, pointer] : unused)
-                    {
-                        freed.push_back(pointer);
-                    }
+                    pool.drop_all(freed);
                 }
-                unused_.clear();
             }
         }
-        const BesideCaptures relaxed;
-        for (void* p : freed)
-        {
-            (void)hipFree(p);
-        }
+        release(freed);
     }
 
   private:
+    struct Pool
+    {
+        Buffers unused;
+        std::size_t total = 0; // bytes of the unused buffers and of those in use
+
+        void drop(Buffers::iterator at, Buffers& freed)
+        {
+            total -= at->first;
+            freed.insert(unused.extract(at));
+        }
+        void drop_all(Buffers& freed)
+        {
+            while (!unused.empty())
+            {
+                drop(unused.begin(), freed);
+            }
+        }
+    };
+
+    static hipError_t allocate(void** pointer, std::size_t bytes)
+    {
+        const BesideCaptures relaxed;
+        const hipError_t status = hipMalloc(pointer, bytes);
+        if (status != hipSuccess)
+        {
+            (void)hipGetLastError(); // not the next launch's error
+        }
+        return status;
+    }
+    static void release(const Buffers& freed)
+    {
+        if (freed.empty())
+        {
+            return;
+        }
+        const BesideCaptures relaxed;
+        for (const auto& [bytes, pointer] : freed)
+        {
+            (void)hipFree(pointer);
+        }
+    }
+
     std::mutex mutex_;
-    std::map<int, std::multimap<std::size_t, void*>> unused_;
+    std::map<int, Pool> pools_;
     std::size_t projections_ = 0;
 };
 
@@ -333,29 +401,45 @@ class ErrorWords
     bool waited_ = false;
 };
 
-// One call's buffer; declared after its ErrorWords, whose check() has waited for the
-// stream unless the call failed.
+// One call's buffer, kept or stream-ordered; declared after its ErrorWords, whose check()
+// has waited for the stream unless the call failed.
 class ProjectionScratch
 {
   public:
-    ProjectionScratch(std::size_t bytes, const ErrorWords& words)
+    ProjectionScratch(std::size_t bytes, const ErrorWords& words, hipStream_t stream)
         : buffer_(projection_buffers().take(bytes)), words_(words)
     {
+        if (!buffer_.pointer())
+        {
+            try
+            {
+                ordered_.emplace(bytes, stream);
+            }
+            catch (const Error&)
+            {
+                projection_buffers().release_unused(buffer_.device);
+                ordered_.emplace(bytes, stream);
+            }
+        }
     }
     ~ProjectionScratch()
     {
         words_.wait();
-        projection_buffers().give(buffer_);
+        if (buffer_.pointer())
+        {
+            projection_buffers().give(buffer_);
+        }
     }
     ProjectionScratch(const ProjectionScratch&) = delete;
     ProjectionScratch& operator=(const ProjectionScratch&) = delete;
     void* get() const
     {
-        return buffer_.pointer;
+        return ordered_ ? ordered_->pointer : buffer_.pointer();
     }
 
   private:
     ProjectionBuffers::Buffer buffer_;
+    std::optional<AsyncScratch> ordered_;
     const ErrorWords& words_;
 };
 
@@ -1085,7 +1169,7 @@ int tsac_hip_linear_apply(const tsac_hip_device_linear* linear, const uint16_t* 
                 errors.check("BF8L activations must be finite");
                 return;
             }
-            ProjectionScratch scratch(rows * K + rows * (K / 256) * 4 + 256, errors);
+            ProjectionScratch scratch(rows * K + rows * (K / 256) * 4 + 256, errors, s);
             auto* q = static_cast<int8_t*>(scratch.get());
             auto* scales =
                 reinterpret_cast<float*>(static_cast<uint8_t*>(scratch.get()) + (rows * K + 255) / 256 * 256);
