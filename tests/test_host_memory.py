@@ -159,3 +159,27 @@ def test_projection_buffers_of_overlapping_calls(host_hip):
     import gc; gc.collect()
     assert hip.host_hip_used() == 0
     """))
+
+
+DAC = """
+geometry = synthetic.Geometry(width=256, heads=2, head_width=128, ffn=512, temporal_layers=1, codebook_layers=1,
+                              latent=256, books=9, channels=1)
+session = native.HipModel(synthetic.random_model(geometry, seed=1)).session()
+model = synthetic.random_dac(channels=1, books=9, seed=1)
+dac = native.HipDac(model)
+launches()
+"""
+
+
+@pytest.mark.parametrize("frames,groups", [(2700, 400), (400, 2700), (20, 60000)])
+def test_analysis_of_very_many_channels(host_hip, frames, groups):
+    """Interleaved PCM whose channels' rows span more than 2 GiB is analysed, chunks long
+    and short: offsets are relative to a workgroup's first frame."""
+    run(host_hip, DAC + f"frames, groups = {frames}, {groups}" + textwrap.dedent("""
+    pcm = np.zeros((frames * 512, groups), np.float32)  # never touched
+    tokens = np.zeros(frames * groups, np.uint16)
+    status = lib.tsac_hip_dac_analyze(session.handle, dac.handle, native._ptr(pcm, ctypes.c_float), frames, groups, 1,
+                                      native._ptr(tokens, ctypes.c_uint16))
+    assert status == 0, lib.tsac_hip_last_error()
+    assert len(launches()) >= groups * 31
+    """))

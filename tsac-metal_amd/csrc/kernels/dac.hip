@@ -70,15 +70,16 @@ __device__ __forceinline__ float snake(float y, float a, bool& finite)
 }
 
 // Rows of a signal through range-checked buffer loads: a lane whose frame is
-// outside the signal gets `outside` as its offset and reads 0. A skipped term and
+// outside the signal gets `outside` as its offset and reads 0 (every other offset is
+// below 2 GiB, which dac_conv checks). A skipped term and
 // an added 0 * w are the same: a sum starts at +0 and no IEEE addition of +0 and a
 // zero, or of opposite finite values, gives -0, so adding a zero of either sign
 // never changes a sum.
 constexpr uint32_t outside = 0x80000000u;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const float* row, int bytes)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const float* row)
 {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row), 0, bytes, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row), 0, 0x7fffffff, 0x00020000);
 }
 __device__ __forceinline__ float row_load(__amdgpu_buffer_rsrc_t row, uint32_t at)
 {
@@ -94,19 +95,12 @@ __device__ __forceinline__ constant_ptr<ConvArgs> arguments()
     return p;
 }
 
-// Byte offset of frame f in a channel's row.
-__device__ __forceinline__ uint32_t frame_offset(const __attribute__((address_space(4))) Strided& s, int f)
+// Byte offset of frame f in a channel's row from frame `from` on (0 where polyphase).
+__device__ __forceinline__ uint32_t frame_offset(const __attribute__((address_space(4))) Strided& s, int f, int from)
 {
     const int phases = s.phases;
-    const long long at = phases > 1 ? (f % phases) * s.phase + (f / phases) * s.frame : f * s.frame;
+    const long long at = phases > 1 ? (f % phases) * s.phase + (f / phases) * s.frame : (f - from) * s.frame;
     return uint32_t(at) * 4u;
-}
-// Bytes of a channel's row of `frames` frames.
-__device__ __forceinline__ int row_bytes(const __attribute__((address_space(4))) Strided& s, int frames)
-{
-    const long long last = s.phases > 1 ? (s.phases - 1) * s.phase + (frames / s.phases - 1) * s.frame
-                                        : (frames - 1) * s.frame;
-    return int((last + 1) * 4);
 }
 
 // LDS-only workgroup barrier: the next stage's global loads stay in flight.
@@ -229,11 +223,18 @@ __global__ __launch_bounds__(conv_threads) __attribute__((amdgpu_waves_per_eu(4,
     constexpr bool uniform_row = across % lanes == 0;
     const int column = thread % across;
     const int row = uniform_row ? __builtin_amdgcn_readfirstlane(thread / across) : thread / across;
-    const int bytes = row_bytes(args->x, args->frames) + (uniform_row ? 0 : int((rows - 1) * channel * 4));
     uint32_t at[steps];
+    // The first frame the tile reads, which its offsets count from: the rows of
+    // interleaved PCM may span more than an offset holds.
+    const auto first_frame = [&](constant_ptr<ConvArgs> now)
+    {
+        const int least = Transposed ? p0 - (taps - 1) : p0 * now->conv.shape.stride - now->conv.shape.padding;
+        return now->x.phases > 1 || least < 0 ? 0 : least;
+    };
     const auto offsets = [&](int tap)
     {
         const auto now = arguments();
+        const int from = first_frame(now);
         const int step = Transposed ? 1 : now->conv.shape.stride;
         const int origin = Transposed ? -tap : tap * now->conv.shape.dilation - now->conv.shape.padding;
         const int frames = now->frames;
@@ -242,11 +243,11 @@ __global__ __launch_bounds__(conv_threads) __attribute__((amdgpu_waves_per_eu(4,
         {
             const int source = (p0 + column + i * across) * step + origin;
             at[i] = source >= 0 && source < frames
-                        ? frame_offset(now->x, source) + (uniform_row ? 0u : uint32_t(row * int(channel)) * 4u)
+                        ? frame_offset(now->x, source, from) + (uniform_row ? 0u : uint32_t(row * int(channel)) * 4u)
                         : outside;
         }
     };
-    const float* const first_row = args->x.data + (uniform_row ? row * channel : 0);
+    const float* const first_row = args->x.data + first_frame(args) * args->x.frame + (uniform_row ? row * channel : 0);
     const float* x = first_row;
     float held[passes][steps];
     // Weights: float4s t, t + conv_threads, ... of the stage's KB x TC.
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(conv_threads) __attribute__((amdgpu_waves_per_eu(4,
         {
             if (KB % rows == 0 || row + p * rows < KB)
             {
-                const __amdgpu_buffer_rsrc_t source = row_buffer(x + p * rows * channel, bytes);
+                const __amdgpu_buffer_rsrc_t source = row_buffer(x + p * rows * channel);
 #pragma unroll
                 for (int i = 0; i < steps; ++i)
                 {
@@ -790,10 +791,15 @@ void dac_conv(const ConvArgs& a, hipStream_t stream)
     require(!s.transposed || s.stride == 2 || s.stride % 4 == 0, "dac convolution: transposed stride");
     require(!a.residual.data || (a.residual.channel == a.out.channel && a.residual.frame == a.out.frame),
             "dac convolution: the residual is laid out as the output");
+    // What a tile of at most `widest` positions reads of a channel, or of polyphase
+    // planes the whole channel.
+    constexpr int widest = 256;
+    const long long reads = s.transposed ? widest + s.kernel / s.stride - 1
+                                         : (widest - 1) * s.stride + (s.kernel - 1) * s.dilation + 1;
     const long long extent = a.x.phases > 1
                                  ? (a.x.phases - 1) * a.x.phase + (a.frames / a.x.phases - 1) * a.x.frame
-                                 : (a.frames - 1) * a.x.frame;
-    require(extent >= 0 && extent < (1ll << 29) - 1, "dac convolution: a channel's frames span 2 GiB");
+                                 : (std::min<long long>(reads, a.frames) - 1) * a.x.frame;
+    require(extent >= 0 && extent < (1ll << 29) - 1, "dac convolution: a tile's frames span 2 GiB");
     const int out_frames = s.output_frames(a.frames);
     require(out_frames > 0, "dac convolution has no output frames");
     const int positions = s.transposed ? (out_frames + s.padding + s.stride - 1) / s.stride : out_frames;
@@ -801,6 +807,7 @@ void dac_conv(const ConvArgs& a, hipStream_t stream)
     const auto launch = [&](auto tile)
     {
         using T = decltype(tile);
+        static_assert(T::positions <= widest);
         require(s.in % T::kb == 0, "dac convolution: inputs are a multiple of the stage");
         const dim3 grid(unsigned((positions + T::positions - 1) / T::positions),
                         unsigned((columns + T::columns - 1) / T::columns));
