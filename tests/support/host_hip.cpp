@@ -16,7 +16,7 @@ namespace
 std::mutex mutex;
 uintptr_t next_address = uintptr_t(1) << 44;
 std::map<uintptr_t, size_t> device; // allocations
-size_t device_total = size_t(288) << 30, device_used = 0;
+size_t device_total = size_t(288) << 30, device_used = 0, largest = ~size_t(0);
 std::map<std::string, long> counts;
 bool pinned_fails = false;
 unsigned fill = 0x4000; // 16-bit value that copies to the host leave
@@ -39,7 +39,7 @@ hipError_t failed(hipError_t e)
 hipError_t allocate(void** p, size_t bytes)
 {
     const std::lock_guard<std::mutex> lock(mutex);
-    if (device_used + bytes > device_total)
+    if (bytes > largest || device_used + bytes > device_total)
     {
         return failed(hipErrorOutOfMemory);
     }
@@ -93,6 +93,10 @@ extern "C"
 void host_hip_total(size_t bytes)
 {
     device_total = bytes;
+}
+void host_hip_largest(size_t bytes) // of one allocation
+{
+    largest = bytes;
 }
 size_t host_hip_used()
 {

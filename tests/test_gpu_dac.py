@@ -163,3 +163,22 @@ def test_convolution_tiles_agree_across_sizes(stereo, mono, synthesis, frames):
             window = np.ascontiguousarray(signal[low * step:high * step])
             short = dac.apply(session, synthesis, window, (high - low) * step).reshape(high - low, -1)
             assert np.array_equal(_bits(short[begin - low:begin - low + count]), _bits(long[begin:begin + count]))
+
+
+@pytest.mark.parametrize("channels", [1, 2])
+def test_equal_chunks_past_the_reference_length(native, stereo, mono, channels):
+    """Recordings longer than one large chunk run in equal chunks (334, 334 and 332 of
+    1,000 frames under a limit of 450): the tokens and samples of one chunk, whichever
+    graph used the session's scratch before."""
+    model, _, session, dac, _, _ = mono if channels == 1 else stereo
+    frames = 1000
+    limited = native.HipDac(model, native.Limits(0, 0, 0, 0, 96 * 512 * (450 + 22)))
+    pcm = _pcm(frames * 512 / 44100, channels, 13, frames)
+    tokens = dac.analyze(session, pcm, frames)
+    assert np.array_equal(limited.analyze(session, pcm, frames), tokens)
+    audio = limited.synthesize(session, tokens, frames)
+    assert np.array_equal(_bits(audio), _bits(dac.synthesize(session, tokens, frames)))
+    assert np.array_equal(limited.analyze(session, pcm, frames), tokens)
+    session.clear()
+    assert np.array_equal(_bits(limited.synthesize(session, tokens, frames)), _bits(audio))
+    limited.close()

@@ -15,6 +15,7 @@ import ctypes, sys
 sys.path.insert(0, {package!r})
 hip = ctypes.CDLL({hip!r}, mode=ctypes.RTLD_GLOBAL)
 hip.host_hip_total.argtypes = [ctypes.c_size_t]
+hip.host_hip_largest.argtypes = [ctypes.c_size_t]
 hip.host_hip_used.restype = ctypes.c_size_t
 hip.host_hip_count.argtypes, hip.host_hip_count.restype = [ctypes.c_char_p], ctypes.c_long
 hip.host_hip_launches.restype = ctypes.c_char_p
@@ -182,4 +183,71 @@ def test_analysis_of_very_many_channels(host_hip, frames, groups):
                                       native._ptr(tokens, ctypes.c_uint16))
     assert status == 0, lib.tsac_hip_last_error()
     assert len(launches()) >= groups * 31
+    """))
+
+
+CHUNKS = DAC + """
+def analyze(frames, groups=1):
+    launches()
+    dac.analyze(session, np.zeros((frames * 512, groups), np.float32), frames, groups)
+    return sum("rvq_encode" in line[0] for line in launches()) // groups  # chunks
+
+def synthesize(frames):
+    launches()
+    dac.synthesize(session, np.zeros(frames * 9, np.uint16), frames)
+    return sum("rvq_decode" in line[0] for line in launches())
+
+base = hip.host_hip_used()
+SLOTS = {False: 3 * 64 * 512 * 4, True: 3 * 96 * 512 * 4}  # bytes a frame
+"""
+
+
+def test_dac_chunks_follow_the_memory(host_hip):
+    """Long recordings run in equal chunks of up to 2,708 latent frames (the default
+    element limit; at most 3,072 by any), in the reference's 400 where an eighth of the
+    device's free memory holds no more."""
+    run(host_hip, CHUNKS + textwrap.dedent("""
+    assert [analyze(n) for n in (1, 400, 401, 2584, 2708, 2709, 8000)] == [1, 1, 1, 1, 1, 2, 3]
+    assert [synthesize(n) for n in (1, 400, 401, 2584, 2708, 2709, 8000)] == [1, 1, 1, 1, 1, 2, 3]
+    wide = native.HipDac(model, native.Limits(0, 0, 0, 0, 1 << 30))
+    launches()
+    wide.analyze(session, np.zeros((3073 * 512, 1), np.float32), 3073)
+    assert sum("rvq_encode" in line[0] for line in launches()) == 2
+    session.clear()
+    hip.host_hip_total(base + GiB)
+    assert analyze(2584) == 7 and synthesize(2584) == 7
+    """))
+
+
+def test_dac_graphs_share_their_scratch(host_hip):
+    """Analysis and synthesis keep one set of slots between them, as large as the larger
+    needs, next to their inputs and outputs."""
+    run(host_hip, CHUNKS + textwrap.dedent("""
+    analyze(2584), synthesize(2584)
+    assert hip.host_hip_used() - base < 2584 * SLOTS[True] + 64 * MiB
+    """))
+
+
+def test_dac_scratch_is_given_back_where_memory_is_short(host_hip):
+    """Slots kept from a call with more memory are freed once they exceed an eighth of what
+    is left, and at once where another of the session's buffers finds no memory; where
+    the memory for a large chunk cannot be had, chunks of 400 frames run."""
+    run(host_hip, CHUNKS + textwrap.dedent("""
+    for frames, chunks in ((2584, 7), (100, 1)):  # by a long call and by a short one
+        hip.host_hip_total(288 * GiB)
+        assert synthesize(2584) == 1
+        hip.host_hip_total(hip.host_hip_used() + 300 * MiB)
+        assert synthesize(frames) == chunks
+        assert hip.host_hip_used() - base < 422 * SLOTS[True] + 64 * MiB
+    session.clear()
+
+    hip.host_hip_total(288 * GiB)
+    assert synthesize(2584) == 1
+    hip.host_hip_total(hip.host_hip_used() + 12 * GiB)
+    assert analyze(2584, groups=2450) == 1  # 12.1 GiB of samples
+    session.clear()
+
+    hip.host_hip_total(288 * GiB)
+    hip.host_hip_largest(200 * MiB)
+    assert synthesize(2584) == 7 and analyze(2584) == 7
     """))

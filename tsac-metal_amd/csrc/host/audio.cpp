@@ -409,28 +409,61 @@ Chunk chunk_at(std::size_t begin, std::size_t frames, std::size_t size, std::siz
     return {begin, count, begin > left_context ? begin - left_context : 0, end + std::min(right_context, frames - end)};
 }
 
-// Latent frames a chunk: the reference's 400 for short signals, else as many as
-// keep the layers of the lowest rates busy, in equal chunks. Those layers have one
-// to eight frames per latent frame, so 400 leave most of the device idle (30 s of
-// stereo, 2,584 frames: analysis and coding 61.5 ms in chunks of 400, 54.6 of 1,292,
-// 51.0 in one; synthesis 91.0, 82.6 and 80.0). The chunk changes no value, only
-// the scratch, `frame_bytes` a frame (3,072 frames: 1.2 GB analysing, 1.8
-// synthesising), which takes at most an eighth of the free device memory.
-std::size_t chunk_frames(std::size_t frames, std::size_t frame_bytes, const Limits& limits)
-{
-    constexpr std::size_t least = 400, most = 3072;
-    std::size_t target = least;
-    if (frames > least)
-    {
-        std::size_t available = 0, total = 0;
-        check_hip(hipMemGetInfo(&available, &total), "hipMemGetInfo");
-        target = std::clamp(available / 8 / frame_bytes, least, most);
-    }
-    const std::size_t longest = audio_chunk_frames(target, limits);
-    const std::size_t chunks = (frames + longest - 1) / longest;
-    return longest <= least ? longest : (frames + chunks - 1) / chunks;
-}
+constexpr std::size_t least_chunk = 400; // the reference's
+
+constexpr const char* slot_names[3] = {"dac.0", "dac.1", "dac.2"};
 } // namespace
+
+// The reference's 400 frames for short signals, else as many as keep the layers of
+// the lowest rates busy, in equal chunks. Those layers have one to eight frames per
+// latent frame, so 400 leave most of the device idle (30 s of stereo, 2,584 frames:
+// analysis and coding 61.5 ms in chunks of 400, 54.6 of 1,292, 51.0 in one; synthesis
+// 91.0, 82.6 and 80.0). The chunk changes no value, only the slots' bytes, at most an
+// eighth of the device memory that is free or held by them; Limits::tensor_elements
+// ends the default chunk at 2,708 frames (1.1 GB analysing, 1.6 synthesising).
+std::size_t Session::plan_chunk(std::size_t frames, std::size_t frame_bytes, std::size_t context, const Limits& limits)
+{
+    constexpr std::size_t most = 3072;
+    const std::size_t least = audio_chunk_frames(least_chunk, limits);
+    std::size_t kept = 0, chunk = least;
+    for (const char* name : slot_names)
+    {
+        kept += arena_.bytes(name);
+    }
+    if (frames <= least_chunk && kept <= frame_bytes * (least_chunk + context))
+    {
+        return chunk;
+    }
+    std::size_t available = 0, total = 0;
+    check_hip(hipMemGetInfo(&available, &total), "hipMemGetInfo");
+    const std::size_t share = (available + kept) / 8;
+    const std::size_t longest =
+        audio_chunk_frames(std::clamp(share / frame_bytes, least_chunk + context, most + context) - context, limits);
+    if (frames > least_chunk && longest > least_chunk)
+    {
+        const std::size_t chunks = (frames + longest - 1) / longest;
+        chunk = (frames + chunks - 1) / chunks;
+    }
+    if (kept > share && kept > frame_bytes * std::min(frames, chunk + context))
+    {
+        release_dac_slots();
+    }
+    return chunk;
+}
+
+std::array<float*, 3> Session::dac_slots(std::size_t floats)
+{
+    return {arena_.get<float>(slot_names[0], floats), arena_.get<float>(slot_names[1], floats),
+            arena_.get<float>(slot_names[2], floats)};
+}
+
+void Session::release_dac_slots()
+{
+    for (const char* name : slot_names)
+    {
+        arena_.release(name);
+    }
+}
 
 // DacAnalysis::apply (src/common/analysis.tpp:150-190) on `samples` frames of
 // `input`: the entry convolution, four stages of three residual units and a
@@ -558,17 +591,17 @@ void Session::dac_apply(const DacModel& dac, bool synthesis, const float* input,
     const std::size_t slot = synthesis ? 96 * hop * frames : 64 * frames;
     auto* d_in = arena_.get<float>("d.in", in_count);
     auto* d_out = arena_.get<float>("d.out", out_count);
-    float* slots[3] = {arena_.get<float>("d.0", slot), arena_.get<float>("d.1", slot), arena_.get<float>("d.2", slot)};
+    const auto slots = dac_slots(slot);
     reset_errors();
     upload_input(d_in, input, in_count * sizeof(float));
     if (synthesis)
     {
         synthesis_graph(dac, Strided{d_in, 1, 1024}, int(frames), Strided{d_out, 1, (long long)channels}, 0,
-                        int(frames * hop), slots);
+                        int(frames * hop), slots.data());
     }
     else
     {
-        analysis_graph(dac, Strided{d_in, 1, (long long)channels}, int(frames), Strided{d_out, 1, 1024}, slots);
+        analysis_graph(dac, Strided{d_in, 1, (long long)channels}, int(frames), Strided{d_out, 1, 1024}, slots.data());
     }
     check_hip(hipMemcpyAsync(output, d_out, out_count * sizeof(float), hipMemcpyDeviceToHost, stream_), "read output");
     check_dsp_errors();
@@ -585,13 +618,28 @@ void Session::analyze(const DacModel& dac, const float* pcm, std::size_t frames,
     {
         return;
     }
-    const std::size_t chunk = chunk_frames(frames, 3 * 64 * hop * sizeof(float), dac.limits());
-    const std::size_t widest = std::min(frames, chunk + 17) * hop;
+    constexpr std::size_t context = 17;
+    std::size_t chunk = plan_chunk(frames, 3 * 64 * hop * sizeof(float), context, dac.limits());
     auto* d_pcm = arena_.get<float>("a.pcm", samples * stride);
     auto* d_tokens = arena_.get<uint16_t>("a.tokens", frames * groups * books);
-    auto* latent = arena_.get<float>("a.latent", 1024 * (widest / hop));
-    float* slots[3] = {arena_.get<float>("a.0", 64 * widest), arena_.get<float>("a.1", 64 * widest),
-                       arena_.get<float>("a.2", 64 * widest)};
+    float* latent = nullptr;
+    std::array<float*, 3> slots;
+    const auto allocate = [&]
+    {
+        const std::size_t widest = std::min(frames, chunk + context);
+        latent = arena_.get<float>("dac.latent", 1024 * widest);
+        slots = dac_slots(64 * hop * widest);
+    };
+    try
+    {
+        allocate();
+    }
+    catch (const Error&)
+    {
+        release_dac_slots();
+        chunk = audio_chunk_frames(least_chunk, dac.limits());
+        allocate();
+    }
     reset_errors();
     upload_input(d_pcm, pcm, samples * stride * sizeof(float));
     for (std::size_t g = 0; g < groups; ++g)
@@ -601,7 +649,7 @@ void Session::analyze(const DacModel& dac, const float* pcm, std::size_t frames,
             const Chunk c = chunk_at(begin, frames, chunk, 8, 9);
             const int n = int(c.right - c.left);
             analysis_graph(dac, Strided{d_pcm + c.left * hop * stride + g * channels, 1, (long long)stride},
-                           n * int(hop), Strided{latent, n, 1}, slots);
+                           n * int(hop), Strided{latent, n, 1}, slots.data());
             rvq_encode(dac.rvq(), int(books), latent + (c.begin - c.left), n, int(c.count),
                        d_tokens + (c.begin * groups + g) * books, int(groups * books), errors_.as<uint32_t>(), stream_);
             begin += c.count;
@@ -627,13 +675,28 @@ void Session::synthesize(const DacModel& dac, const uint16_t* tokens, std::size_
     {
         require(tokens[i] < 1024, "token above 1023: outside the 1024-symbol alphabet");
     }
-    const std::size_t chunk = chunk_frames(frames, 3 * 96 * hop * sizeof(float), dac.limits());
-    const std::size_t widest = std::min(frames, chunk + 22);
+    constexpr std::size_t context = 22;
+    std::size_t chunk = plan_chunk(frames, 3 * 96 * hop * sizeof(float), context, dac.limits());
     auto* d_tokens = arena_.get<uint16_t>("y.tokens", frames * groups * books);
     auto* d_pcm = arena_.get<float>("y.pcm", frames * hop * stride);
-    auto* latent = arena_.get<float>("y.latent", 1024 * widest);
-    float* slots[3] = {arena_.get<float>("y.0", 96 * hop * widest), arena_.get<float>("y.1", 96 * hop * widest),
-                       arena_.get<float>("y.2", 96 * hop * widest)};
+    float* latent = nullptr;
+    std::array<float*, 3> slots;
+    const auto allocate = [&]
+    {
+        const std::size_t widest = std::min(frames, chunk + context);
+        latent = arena_.get<float>("dac.latent", 1024 * widest);
+        slots = dac_slots(96 * hop * widest);
+    };
+    try
+    {
+        allocate();
+    }
+    catch (const Error&)
+    {
+        release_dac_slots();
+        chunk = audio_chunk_frames(least_chunk, dac.limits());
+        allocate();
+    }
     reset_errors();
     upload_input(d_tokens, tokens, frames * groups * books * 2);
     for (std::size_t g = 0; g < groups; ++g)
@@ -648,7 +711,7 @@ void Session::synthesize(const DacModel& dac, const uint16_t* tokens, std::size_
             const int first = int((c.begin - c.left) * hop);
             synthesis_graph(dac, Strided{latent, n, 1},
                             n, Strided{d_pcm + c.left * hop * stride + g * channels, 1, (long long)stride}, first,
-                            first + int(c.count * hop), slots);
+                            first + int(c.count * hop), slots.data());
             begin += c.count;
         }
     }
@@ -707,6 +770,10 @@ void Session::check_dsp_errors()
     check_hip(hipMemcpyAsync(pinned_errors_.as<uint32_t>(), errors_.get(), 12, hipMemcpyDeviceToHost, stream_),
               "read error words");
     check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+    for (const char* name : slot_names)
+    {
+        arena_.spare(name);
+    }
     require(!pinned_errors_.as<uint32_t>()[0], "nonfinite DSP value");
 }
 } // namespace tsac_hip

@@ -145,13 +145,45 @@ bool PinnedBuffer::try_reserve(std::size_t bytes)
 
 void* Arena::get(const std::string& name, std::size_t bytes)
 {
-    auto& buffer = buffers_[name];
-    if (buffer.bytes() < bytes)
+    Named& n = buffers_[name];
+    n.spare = false;
+    if (n.buffer.bytes() < bytes)
     {
-        buffer = DeviceBuffer();
-        buffer = DeviceBuffer(align_up(std::max<std::size_t>(bytes, 256), 256));
+        bytes = align_up(std::max<std::size_t>(bytes, 256), 256);
+        n.buffer = DeviceBuffer();
+        try
+        {
+            n.buffer = DeviceBuffer(bytes);
+        }
+        catch (const Error&)
+        {
+            for (auto& [other, named] : buffers_)
+            {
+                if (named.spare)
+                {
+                    named = Named();
+                }
+            }
+            n.buffer = DeviceBuffer(bytes);
+        }
     }
-    return buffer.get();
+    return n.buffer.get();
+}
+
+std::size_t Arena::bytes(const std::string& name) const
+{
+    const auto found = buffers_.find(name);
+    return found == buffers_.end() ? 0 : found->second.buffer.bytes();
+}
+
+void Arena::spare(const std::string& name)
+{
+    buffers_[name].spare = true;
+}
+
+void Arena::release(const std::string& name)
+{
+    buffers_.erase(name);
 }
 
 // ---------------------------------------------------------------- model

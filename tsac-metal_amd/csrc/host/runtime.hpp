@@ -106,13 +106,22 @@ public:
     {
         return static_cast<T*>(get(name, count * sizeof(T)));
     }
+    std::size_t bytes(const std::string& name) const;
+    // An idle buffer that is freed where another one finds no memory, until its next get().
+    void spare(const std::string& name);
+    void release(const std::string& name);
     void clear()
     {
         buffers_.clear();
     }
 
 private:
-    std::map<std::string, DeviceBuffer> buffers_;
+    struct Named
+    {
+        DeviceBuffer buffer;
+        bool spare = false;
+    };
+    std::map<std::string, Named> buffers_;
 };
 
 struct LinearHost
@@ -247,6 +256,12 @@ private:
     struct Stepwise;
     void check_errors();
     void check_dsp_errors();
+    // Latent frames a chunk of a DAC graph whose slots take `frame_bytes` a frame, for
+    // `frames` with `context` frames around a chunk. Frees slots that are too large now.
+    std::size_t plan_chunk(std::size_t frames, std::size_t frame_bytes, std::size_t context, const Limits& limits);
+    // The graphs' three activation slots, one set for all of a session's graphs.
+    std::array<float*, 3> dac_slots(std::size_t floats);
+    void release_dac_slots();
     void analysis_graph(const DacModel& dac, Strided input, int samples, Strided output, float* const* slots);
     void synthesis_graph(const DacModel& dac, Strided input, int frames, Strided output, int first, int last,
                          float* const* slots);
