@@ -635,6 +635,49 @@ def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, 
         start += length
 
 
+@pytest.mark.parametrize("sequences,length", [(4_300_000, 1), (300_000, 20)])
+def test_attention_causal_of_very_many_sequences(torch, native, sequences, length):
+    """More (sequence, head) pairs than one launch takes. The sequences lie over the same
+    few rows, so that each of them gives what a call of one of each gives."""
+    heads, hw, starts = 16, 64, 61
+    rng = np.random.default_rng(length)
+    w = heads * hw
+    qkv = dev(torch, bf16_bits(rng.standard_normal((starts * length, 3 * w)).astype(np.float32)))
+    scale = np.float32(1 / np.sqrt(hw))
+
+    def run(n):
+        start = (torch.arange(n, device="cuda") % starts * length).to(torch.int32)
+        lengths, replay = torch.full_like(start, length), torch.zeros_like(start)
+        if n > starts:
+            # the last of them alone, where an earlier slice does not reach
+            start[-1], qkv_last = starts * length, torch.cat([qkv, qkv[:length]])
+        else:
+            qkv_last = qkv
+        out = torch.zeros((qkv_last.shape[0], w), dtype=torch.int16, device="cuda")
+        native.attention_causal(qkv_last, heads, hw, start, lengths, replay, n, length, None, scale, out)
+        return host(out)
+
+    few, many = run(starts), run(sequences)
+    assert np.array_equal(many[:starts * length], few)
+    assert np.array_equal(many[starts * length:], few[:length])
+
+
+def test_attention_causal_with_a_loose_bound(torch, native):
+    """max_length bounds the lengths; tiles past a sequence's end do nothing, however many."""
+    heads, hw, lengths = 2, 64, [130, 17, 64, 1]
+    rng = np.random.default_rng(3)
+    w, rows = heads * hw, sum(lengths)
+    qkv = dev(torch, bf16_bits(rng.standard_normal((rows, 3 * w)).astype(np.float32)))
+    starts = dev(torch, np.cumsum([0] + lengths[:-1]).astype(np.int32))
+    args = (heads, hw, starts, dev(torch, np.array(lengths, np.int32)), dev(torch, np.zeros(4, np.int32)), 4)
+    tight = empty(torch, (rows, w), torch.int16)
+    native.attention_causal(qkv, *args, 130, None, np.float32(0.125), tight)
+    for bound in (2_200_000, 4_194_240):
+        loose = empty(torch, (rows, w), torch.int16)
+        native.attention_causal(qkv, *args, bound, None, np.float32(0.125), loose)
+        assert np.array_equal(host(loose), host(tight)), bound
+
+
 @pytest.mark.parametrize("k", [256, 512, 1024, 2048, 4096])
 @pytest.mark.parametrize("columns", range(1, 9))
 def test_qlinear_quantises_in_the_gemv(torch, native, oracle, k, columns):

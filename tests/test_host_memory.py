@@ -251,3 +251,33 @@ def test_dac_scratch_is_given_back_where_memory_is_short(host_hip):
     hip.host_hip_largest(200 * MiB)
     assert synthesize(2584) == 7 and analyze(2584) == 7
     """))
+
+
+@pytest.mark.parametrize("sequences,heads,longest", [(1, 1, 2_200_000), (1, 1, 4_194_240), (3, 2, 1_100_000), (2, 1, 65536 * 8),
+                                                     (4_300_000, 16, 1), (16_000_000, 16, 12), (5_500_000, 16, 20),
+                                                     (4_300_000, 16, 65), (1, 65535, 300), (2_000_000, 1, 17)])
+@pytest.mark.parametrize("width", [64, 128])
+def test_causal_attention_launches_any_size(host_hip, sequences, heads, longest, width):
+    """Every (sequence, head, query) has a workgroup, in launches within the limits of a grid."""
+    run(host_hip, f"sequences, heads, longest, width = {sequences}, {heads}, {longest}, {width}" + textwrap.dedent("""
+    status = lib.tsac_hip_attention_causal(1 << 44, heads, width, 1 << 45, 1 << 46, 1 << 47, sequences, longest, None,
+                                           1.0, 1 << 48, None)
+    assert status == 0, lib.tsac_hip_last_error()
+    pairs = 0
+    for name, x, y, z, threads in launches():
+        if "short_kernel" in name:
+            pairs += int(x) * int(threads) // 64  # a wave each, up to 3 to spare
+        else:
+            pairs += int(x)
+            queries = int(name.split("Li")[3].split("E")[0])
+            assert int(y) * int(z) * queries >= longest
+    assert sequences * heads <= pairs <= sequences * heads + 3 * len(launches() or [0]) + 3 * 64
+    """))
+
+
+def test_causal_attention_refuses_no_heads(host_hip):
+    run(host_hip, """
+    for longest in (1, 100):
+        assert lib.tsac_hip_attention_causal(1 << 44, 0, 64, 1 << 45, 1 << 46, 1 << 47, 1, longest, None, 1.0, 1 << 48,
+                                             None) != 0
+    """)

@@ -532,8 +532,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
     __shared__ Shared shared;
     const int sequence = blockIdx.x / heads, head = blockIdx.x % heads;
     const int length = sequence_length[sequence];
-    // The longest histories first.
-    const int q0 = int(gridDim.y - 1 - blockIdx.y) * queries;
+    // The longest histories first; z takes the tiles past a grid's reach along y.
+    const int q0 = int(gridDim.z * gridDim.y - 1 - (blockIdx.z * gridDim.y + blockIdx.y)) * queries;
     if (q0 >= length)
     {
         return;
@@ -1266,16 +1266,22 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
         return;
     }
     require(head_width == 64 || head_width == 128, "attention: head width must be 64 or 128");
-    require(sequences * heads < (std::size_t(1) << 31), "attention: too many sequences");
+    require(heads > 0 && heads < (std::size_t(1) << 22) && max_length < (std::size_t(1) << 30),
+            "attention: heads or rows out of range");
+    // A launch takes so many sequences that its work-items along x stay below 2^32.
+    const std::size_t slice = (std::size_t(1) << 22) / heads;
     if (max_length <= short_rows)
     {
-        const std::size_t pairs = sequences * heads;
         const auto kernel = head_width == 64 ? (rotations ? short_kernel<64, true> : short_kernel<64, false>)
                                              : (rotations ? short_kernel<128, true> : short_kernel<128, false>);
-        kernel<<<unsigned((pairs + short_waves - 1) / short_waves), 64 * short_waves, 0, stream>>>(
-            qkv, int(width), sequence_start, sequence_length, sequence_replay, rotations, int(heads), int(pairs), scale,
-            out);
-        check_hip(hipGetLastError(), "attention prefill launch");
+        for (std::size_t first = 0; first < sequences; first += slice)
+        {
+            const std::size_t pairs = std::min(slice, sequences - first) * heads;
+            kernel<<<unsigned((pairs + short_waves - 1) / short_waves), 64 * short_waves, 0, stream>>>(
+                qkv, int(width), sequence_start + first, sequence_length + first, sequence_replay + first, rotations,
+                int(heads), int(pairs), scale, out);
+            check_hip(hipGetLastError(), "attention prefill launch");
+        }
         return;
     }
     // Waves and queries of a workgroup, by the blocks of the longest history and by how
@@ -1305,9 +1311,17 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     const auto tiles = [&](std::size_t queries) { return sequences * heads * ((max_length + queries - 1) / queries); };
     const auto launch = [&](auto rotary, auto plain, int waves, std::size_t queries)
     {
-        const dim3 grid(unsigned(sequences * heads), unsigned((max_length + queries - 1) / queries));
-        (rotations ? rotary : plain)<<<grid, 64 * waves, 0, stream>>>(
-            qkv, int(width), sequence_start, sequence_length, sequence_replay, rotations, int(heads), scale, out);
+        constexpr std::size_t reach = 65535;
+        const std::size_t columns = (max_length + queries - 1) / queries, layers = (columns + reach - 1) / reach;
+        for (std::size_t first = 0; first < sequences; first += slice)
+        {
+            const dim3 grid(unsigned(std::min(slice, sequences - first) * heads),
+                            unsigned((columns + layers - 1) / layers), unsigned(layers));
+            (rotations ? rotary : plain)<<<grid, 64 * waves, 0, stream>>>(
+                qkv, int(width), sequence_start + first, sequence_length + first, sequence_replay + first, rotations,
+                int(heads), scale, out);
+            check_hip(hipGetLastError(), "attention prefill launch");
+        }
     };
     const auto by_width = [&](auto head)
     {
@@ -1336,6 +1350,5 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
         }
     };
     head_width == 64 ? by_width(std::integral_constant<int, 64>{}) : by_width(std::integral_constant<int, 128>{});
-    check_hip(hipGetLastError(), "attention prefill launch");
 }
 } // namespace tsac_hip
