@@ -15,6 +15,7 @@ DRIVER = r"""
 #include <cstdio>
 #include <cstring>
 #include <random>
+#include <sys/resource.h>
 using namespace tsac_hip;
 
 static uint32_t byte_crc(const std::vector<uint16_t>& tokens)
@@ -91,6 +92,19 @@ int main()
         {
             return 2;
         }
+    }
+    // The coder of the largest recording by default (64 Mi symbols) touches what it writes.
+    SymbolEncoder large(std::size_t(64) << 20);
+    uint16_t even[16];
+    std::fill(even, even + 16, uint16_t(16384));
+    large.put(even, 5);
+    large.finish();
+    rusage usage;
+    getrusage(RUSAGE_SELF, &usage);
+    if (usage.ru_maxrss > 256 * 1024)
+    {
+        std::printf("%ld KiB resident\n", usage.ru_maxrss);
+        return 3;
     }
     return 0;
 }
