@@ -551,14 +551,19 @@ def test_calibration_probes(torch, native):
 @pytest.mark.parametrize("heads,hw", [(16, 64), (4, 128)])
 @pytest.mark.parametrize("lengths,kind", [([65, 31, 33, 64, 1] * 8, "normal"), ([330], "normal"), ([129, 96], "spread"),
                                           ([100], "dead infinity"), ([70], "zeros"), ([65], "tiny"), ([12] * 9, "normal"),
-                                          ([1, 16, 15, 2, 7], "spread"), ([9, 16], "zeros"), ([16], "tiny")])
+                                          ([1, 16, 15, 2, 7], "spread"), ([9, 16], "zeros"), ([16], "tiny"),
+                                          ([12, 16, 1, 7, 2], "rotated"), ([65, 31, 8], "rotated")])
 def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, kind):
-    """The causal kernel's own choices: 4 or 8 waves by the grid, edges of its 32-query
-    and 64-key tiles, scores more than 87 below the maximum (where weights and their
-    sums meet subnormals), and the last block's dead keys, whose values may be
-    infinite, and whose terms must not turn a zero sum's sign."""
+    """The causal kernels' own choices: sequences of at most 16 rows and longer ones, edges
+    of the query and 64-key tiles, scores more than 87 below the maximum (where weights
+    and their sums meet subnormals), and the last block's dead keys, whose values may be
+    infinite, and whose terms must not turn a zero sum's sign; replay counts of none,
+    some, all and more than all of a sequence's rows."""
     rng = np.random.default_rng(sum(lengths) + hw)
     w, rows = heads * hw, sum(lengths)
+    replays = [(0, n // 2, n, n + 9, 1)[i % 5] for i, n in enumerate(lengths)]
+    if len(lengths) == 1:
+        replays = [lengths[0] // 2]
     qkv = rng.standard_normal((rows, 3 * w)).astype(np.float32)
     if kind == "spread":
         qkv[:, :w] *= 60
@@ -574,14 +579,21 @@ def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, ki
     starts = np.cumsum([0] + lengths[:-1]).astype(np.int32)
     scale = np.float32(1 / np.sqrt(hw))
     out = empty(torch, (rows, w), torch.int16)
+    rotations = bf16_bits(rng.uniform(-1, 1, (max(lengths), hw)).astype(np.float32)) if kind == "rotated" else None
     native.attention_causal(dev(torch, qkv), heads, hw, dev(torch, starts), dev(torch, np.array(lengths, np.int32)),
-                            dev(torch, np.zeros(len(lengths), np.int32)), len(lengths), max(lengths), None, scale, out)
+                            dev(torch, np.array(replays, np.int32)), len(lengths), max(lengths),
+                            dev(torch, rotations) if kind == "rotated" else None, scale, out)
     got = host(out)
-    for start, length in list(zip(starts, lengths))[:5]:
+    for start, length, replay in list(zip(starts, lengths, replays))[:5]:
         seq = qkv[start:start + length]
         q, k, v = seq[:, :w].copy(), seq[:, w:2 * w].copy(), seq[:, 2 * w:].copy()
+        if kind == "rotated":
+            for part in (q, k):
+                for t in range(length):
+                    for h in range(0, w, hw):
+                        part[t, h:h + hw] = oracle.rotary(part[t, h:h + hw], rotations[t])
         for t in range(length):
-            expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, False)
+            expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, t < replay)
             finite = np.isfinite(bf16_float(expected))
             assert np.array_equal(got[start + t][finite], expected[finite]), (length, t)
             assert not np.isfinite(bf16_float(got[start + t][~finite])).any()
@@ -595,9 +607,11 @@ def test_attention_causal_branches(torch, native, oracle, heads, hw, lengths, ki
 def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, pairs, kind):
     """Every choice of waves and queries a workgroup, by the count of (sequence, head)
     pairs: the same sequences again and again equal the first ones, which equal the
-    oracle; rotated in the kernel, they equal a launch of one set."""
+    oracle; rotated in the kernel, they equal a launch of one set. Some sequences have
+    replayed rows, which round the values of queries below 64."""
     rng = np.random.default_rng(sum(lengths) + hw)
     w, rows, sets = heads * hw, sum(lengths), max(1, pairs // (heads * len(lengths)))
+    replays = [(40, 0, length + 1, 5)[i % 4] for i, length in enumerate(lengths)]
     qkv = rng.standard_normal((rows, 3 * w)).astype(np.float32)
     if kind == "spread":
         qkv[:, :w] *= 60
@@ -616,7 +630,7 @@ def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, 
         starts = np.cumsum(np.concatenate([[0], many[:-1]])).astype(np.int32)
         out = empty(torch, (rows * n, w), torch.int16)
         native.attention_causal(dev(torch, np.tile(qkv, (n, 1))), heads, hw, dev(torch, starts), dev(torch, many),
-                                dev(torch, np.zeros(len(many), np.int32)), len(many), max(lengths),
+                                dev(torch, np.array(replays * n, np.int32)), len(many), max(lengths),
                                 dev(torch, rotations) if rotated else None, scale, out)
         return host(out).reshape(n, rows, w)
 
@@ -624,11 +638,11 @@ def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, 
     got = run(sets, False)
     assert np.array_equal(got, np.tile(got[:1], (sets, 1, 1)))
     start = 0
-    for length in lengths:
+    for length, replay in zip(lengths, replays):
         seq = qkv[start:start + length]
         q, k, v = seq[:, :w].copy(), seq[:, w:2 * w].copy(), seq[:, 2 * w:].copy()
         for t in range(length):
-            expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, False)
+            expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, t < replay)
             finite = np.isfinite(bf16_float(expected))
             assert np.array_equal(got[0, start + t][finite], expected[finite]), (length, t)
             assert not np.isfinite(bf16_float(got[0, start + t][~finite])).any()
@@ -737,6 +751,11 @@ def test_layer_norm_of_many_rows(torch, native, oracle, width):
     for r in range(0, rows, 683):
         native.layer_norm(dev(torch, x[r:r + 683]), min(683, rows - r), width, gain, bias, few[r:r + 683])
     assert np.array_equal(host(many), host(few))
+    # at addresses that are multiples of two only, and in place
+    shifted = [torch.empty(t.numel() + 1, dtype=torch.int16, device="cuda")[1:].copy_(t.flatten())
+               for t in (dev(torch, x), gain, bias)]
+    native.layer_norm(shifted[0], rows, width, shifted[1], shifted[2], shifted[0])
+    assert np.array_equal(host(shifted[0]).reshape(rows, width), host(few))
 
 
 @pytest.mark.parametrize("k", [256, 512, 1024, 2048, 4096])
