@@ -501,18 +501,22 @@ template <int HW, int W, int queries> struct PrefillShared
 // ascending block order: a wave waits for its block's turn, which the wave of the
 // block before passes on, so the first block's wave never waits and every wait ends.
 //
-// Bound by VALU issue: 59-70 T fma/s on register operands for the whole chip (the
-// chains over coordinates and keys leave no room for matrix instructions), one
-// instruction per 4.3 cycles from one wave, which makes a block 60 k cycles and the
-// longest query tile's rounds the floor of a short launch. Tiles of 64 queries (8 x 8
-// sums a lane, 13% fewer instructions) made those rounds twice as long: 160 us against
-// 136 for 16 heads of 64 below. One workgroup walking a tile's blocks one after the other
-// with 4 x 4 sums a thread (before) was bound by its LDS reads and barriers. Four
-// waves per SIMD (128 registers) spill and gain nothing. Measured on 3 sequences of
-// 861 rows, before and now: 16 heads of 64 244 -> 136 us, 4 heads of 128 287 -> 88 us;
-// of 2,580 rows 1,222 -> 910 (819 unrotated, with 16 queries) and 942 -> 494. 8 and 16 queries (the launch says when)
-// shorten a block's chain: 4 sequences of 64 rows 15 -> 9.4 and 23 -> 16 us (32 queries:
-// 19 and 34), 4 of 120 rows 27 -> 18 and 41 -> 16.
+// Bound by the issue of the waves that are resident: the chains over coordinates and
+// keys leave no room for matrix instructions, and a wave issues one VALU instruction per
+// 4 cycles at most (two waves of a SIMD issue side by side: 59-70 T fma/s for the whole
+// chip on register operands). Counters of 3 sequences of 861 rows, 16 heads of 64 (4 x 32):
+// 7,500 VALU instructions a block, 4,096 of them the chains' fmas, in 50 k cycles; a wave
+// issues one in 60% of its 4-cycle slots and waits for memory or LDS in 21%, and a
+// SIMD holds 1.45 waves on average, so that the launch reaches 44% of what two waves a SIMD
+// issue. A block's time makes the longest query tile's rounds the floor of a short launch.
+// Tiles of 64 queries (8 x 8 sums a lane, 13% fewer instructions) made those rounds twice
+// as long: 160 us against 136. Four waves per SIMD (128 registers) spill and gain nothing.
+// One workgroup walking a tile's blocks one after the other with 4 x 4 sums a thread
+// (before) was bound by its LDS reads and barriers. us by events around repeated
+// launches, rotated, before and now, 16 heads of 64 | 4 of 128:
+//   861 rows x 3 sequences  232 -> 120 | 287 -> 81        64 x 4   15.2 -> 9.2 | 23 -> 15.6
+//   2,580 x 3              1168 -> 820 | 931 -> 440      120 x 4   27 -> 18    | 42 -> 16
+//   2,580 x 1               602 -> 296 | 835 -> 205      300 x 2   61 -> 38    | 96 -> 28
 template <int HW, int W, int queries, bool Rotary>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) void prefill_kernel(
     const uint16_t* __restrict__ qkv, int width, const int* __restrict__ sequence_start,
@@ -992,8 +996,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
 // empty state by the recurrence all the same.
 //
 // Bound by HBM: each row of the projection is read once and each output written once.
-// 2,580 sequences of 12 rows, 16 heads of 64 (253 MB): 638 us on the tiled kernel above,
-// whose waves each take a whole 64-key block, 85 here (3.0 TB/s); 4 heads of 128, 39.
+// 2,580 sequences of 12 rows, 16 heads of 64 (253 MB): 567 us with 64 queries a workgroup,
+// 79 here (3.2 TB/s); 4 heads of 128 326 and 36. (On the tiled kernel above, whose waves
+// each take a whole 64-key block, 638 and not measured.)
 constexpr int short_rows = 16, short_waves = 4;
 
 template <int HW, bool Rotary>
@@ -1289,18 +1294,37 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     // the chain of a block (8 queries: a quarter of the sums a lane, and its loads wait
     // for memory once), which is the time of a launch that leaves units idle; large ones
     // read and rotate a key for more queries; more waves take more blocks at a time, and
-    // are idle slots where there are none. us, waves x queries, 16 heads of 64 | 4 of 128:
-    //   rows x sequences       1x8   4x8   8x8  1x16  2x16  4x32 |  1x8   4x8   8x8  1x16  2x16  4x32 (8x32 from 300 x 2 on)
-    //   64 x 4                 9.5   9.5    15  13.9  13.3  19.2 | 15.7  15.5  15.5  24.0  23.3  33.5
-    //   64 x 64                 38    52   220    28    32    40 |   21    32    98    26    24    35
-    //   64 x 1000              580   827  3763   369   406   591 |  263   364  1629   193   223   352
-    //   120 x 4                 17    18    31    25    16    21 |   28    16    16    43    24    35
-    //   120 x 100              152   292   735   105   116   203 |   74   133   325    69    64   111
-    //   300 x 2                 37    29    43    57    34    38 |   65    29    29   101    63    38
-    //   430 x 1                 50    27    37    78    45    27 |   91    30    21   141    83    44
-    //   430 x 20               277   402   648   176   185   258 |  146   184   277   146   108   131
-    //   862 x 3                161   194   257   154   115   120 |  183    94   123   286   146    82
-    //   2580 x 1               457   473   551   445   321   297 |  529   235   260   826   423   205
+    // are idle slots where there are none. us by events around repeated rotated launches,
+    // waves x queries, the launched one marked (16 heads of 64, then 4 of 128):
+    //   rows x sequences    1x8    4x8    8x8   1x16   2x16   4x32   8x32
+    //   64 x 4             9.6*    9.6     15     14     13     19     19
+    //   64 x 64             40     53    222    30*     33     41    131
+    //   64 x 1000          577    831   3773   380*    401    592   2150
+    //   120 x 4             17    18*     31     25     16     21     21
+    //   120 x 100          153    293    737    109   115*    203    457
+    //   256 x 3             31     31     51     47     29    26*     40
+    //   300 x 2             37     29     44     56     34     35    38*
+    //   300 x 4             41     49     86     56     35    40*     61
+    //   430 x 1             49    27*     37     76     45     39     27
+    //   430 x 20           276    402    653    176   184*    257    390
+    //   862 x 3            162    194    258    153    114   120*    160
+    //   2580 x 1           456    473    552    443    319   298*    338
+    //   2580 x 3          1294   1414   1650    834   827*    848    979
+    //   64 x 4           15.5*     15     15     24     23     34     33
+    //   64 x 64            21*     31     97     26     24     34     60
+    //   64 x 1000          270    360   1609   207*    222    349    956
+    //   120 x 4             28    16*     16     43     25     35     35
+    //   120 x 100           78    133    321     71    64*    109    219
+    //   256 x 3             54    21*     30     83     46     39     38
+    //   300 x 2             65     29    28*    100     63     61     39
+    //   430 x 1             90     30    21*    140     83     67     43
+    //   430 x 20           146    183    276    147   107*    129    183
+    //   862 x 3            183     93    122    284    147    126    81*
+    //   2580 x 1           530    234    259    827    428    328   206*
+    //   2580 x 3           692    659    752    841    547   441*    442
+    // The lines are drawn through tile counts and do not take every row's best: of 64-wide
+    // heads 300 x 2 (1,216 tiles of 8, past the 4 x 8 line at 1,024) would take 29 us on 4 x 8,
+    // 120 x 4 and 300 x 4 16 and 35 on 2 x 16.
     const std::size_t units = std::size_t(compute_units());
     constexpr std::integral_constant<int, 1> one;
     constexpr std::integral_constant<int, 2> two;

@@ -87,7 +87,7 @@ struct ConvArgs
     Strided activated;
     const float* alpha = nullptr;
     uint32_t* error = nullptr;
-    // Output frames outside [first, last) are neither computed nor stored.
+    // Output frames outside [first, last) are not stored, and their values not checked.
     int first = 0, last = 1 << 30;
 };
 

@@ -145,8 +145,8 @@ void launch_quantize(const uint16_t* x, std::size_t rows, Prologue prologue, con
     const dim3 grid(unsigned((rows + rows_per_block - 1) / rows_per_block)), block(256);
     switch (prologue)
     {
-    case Prologue::none: // bf8l_rows_kernel and quantize_tiles_kernel
-        break;
+    case Prologue::none:
+        throw Error("quantize: rows without a prologue have kernels of their own");
     case Prologue::layer_norm:
         quantize_kernel<V, Prologue::layer_norm><<<grid, block, 0, stream>>>(
             x, int(rows), gain, bias, q, scales, normalized, error, padded_rows);
