@@ -649,6 +649,40 @@ def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, 
         start += length
 
 
+@pytest.mark.parametrize("heads,hw,lengths,sequences", [(8, 64, [256, 250, 193], 480), (8, 64, [384, 330], 236), (8, 64, [200, 70, 64, 1], 800),
+                                                        (8, 64, [65, 64, 30], 900), (4, 128, [96, 65, 7], 1200)])
+def test_attention_causal_of_full_devices(torch, native, oracle, heads, hw, lengths, sequences):
+    """Launches that fill the device with workgroups of one wave (of 32 queries for the first
+    set on 256 compute units, two waves for the second, of 16 for the others): the
+    sequences lie over the rows of the first few, which equal the oracle."""
+    rng = np.random.default_rng(sum(lengths))
+    w, rows, n = heads * hw, sum(lengths), len(lengths)
+    qkv = bf16_bits(rng.standard_normal((rows, 3 * w)).astype(np.float32))
+    qkv[5, 2 * w:] = bf16_bits(np.zeros(w, np.float32))
+    starts = np.resize(np.cumsum([0] + lengths[:-1]), sequences).astype(np.int32)
+    replays = [(40, 0, length + 1, 5)[i % 4] for i, length in enumerate(lengths)]
+    rotations = bf16_bits(rng.uniform(-1, 1, (max(lengths), hw)).astype(np.float32))
+    scale = np.float32(1 / np.sqrt(hw))
+    for rotated in (True, False):
+        out = empty(torch, (rows, w), torch.int16)
+        native.attention_causal(dev(torch, qkv), heads, hw, dev(torch, starts),
+                                dev(torch, np.resize(lengths, sequences).astype(np.int32)),
+                                dev(torch, np.resize(replays, sequences).astype(np.int32)), sequences, max(lengths),
+                                dev(torch, rotations) if rotated else None, scale, out)
+        got = host(out)
+        for start, length, replay in zip(starts[:n], lengths, replays):
+            seq = qkv[start:start + length]
+            q, k, v = seq[:, :w].copy(), seq[:, w:2 * w].copy(), seq[:, 2 * w:].copy()
+            if rotated:
+                for part in (q, k):
+                    for t in range(length):
+                        for h in range(0, w, hw):
+                            part[t, h:h + hw] = oracle.rotary(part[t, h:h + hw], rotations[t])
+            for t in range(length):
+                expected = oracle.attention(q[t], k[:t + 1], v[:t + 1], heads, hw, scale, t < replay)
+                assert np.array_equal(got[start + t], expected), (rotated, length, t)
+
+
 @pytest.mark.parametrize("sequences,length", [(4_300_000, 1), (300_000, 20)])
 def test_attention_causal_of_very_many_sequences(torch, native, sequences, length):
     """More (sequence, head) pairs than one launch takes. The sequences lie over the same
