@@ -77,10 +77,10 @@ hipError_t copy(void* to, size_t bytes, hipMemcpyKind kind)
 {
     if (kind == hipMemcpyDeviceToHost)
     {
-        // A call's error words are 12 bytes, and none is set.
+        // A call's error words are at most 12 bytes, and none is set.
         for (size_t i = 0; i < bytes / 2; ++i)
         {
-            static_cast<uint16_t*>(to)[i] = bytes == 12 ? 0 : uint16_t(fill);
+            static_cast<uint16_t*>(to)[i] = bytes <= 12 ? 0 : uint16_t(fill);
         }
     }
     return hipSuccess;

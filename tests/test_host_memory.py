@@ -281,3 +281,23 @@ def test_causal_attention_refuses_no_heads(host_hip):
         assert lib.tsac_hip_attention_causal(1 << 44, 0, 64, 1 << 45, 1 << 46, 1 << 47, 1, longest, None, 1.0, 1 << 48,
                                              None) != 0
     """)
+
+
+def test_operators_without_page_locked_memory(host_hip):
+    """The calls that report a nonfinite input run without page-locked memory too."""
+    run(host_hip, """
+    hip.host_hip_pinned_fails(1)
+    linear = native.DeviceLinear(np.zeros((256, 256), np.int8), np.ones((1, 256), np.float32), np.zeros(256, np.float32))
+    used = hip.host_hip_used()
+    a, b, c = 1 << 44, 1 << 45, 1 << 46
+    for rows in (3, 100, 5000):
+        assert lib.tsac_hip_linear_apply(linear.handle, a, rows, b, native.PATH_AUTO, None) == 0, lib.tsac_hip_last_error()
+        assert lib.tsac_hip_bf8l(a, rows, 256, b, c, None) == 0, lib.tsac_hip_last_error()
+        assert lib.tsac_hip_bf8l_tiles(a, rows, 256, b, c, None) == 0, lib.tsac_hip_last_error()
+        assert lib.tsac_hip_softmax(a, rows, 256, b, None) == 0, lib.tsac_hip_last_error()
+    after = counts()
+    assert after["hipMallocAsync"] == after["hipFreeAsync"] == 12
+    hip.host_hip_pinned_fails(0)
+    assert lib.tsac_hip_softmax(a, 3, 256, b, None) == 0
+    assert counts() == after
+    """)

@@ -331,7 +331,8 @@ ProjectionBuffers& projection_buffers()
 
 // The error words of one call, in page-locked host memory that its kernels store to:
 // nothing to clear on the device or to copy back. Words are reused; a block of 64
-// pairs is added where more calls overlap.
+// pairs is added where more calls overlap. Where page-locked memory is short, a word of
+// the call's own on the device, cleared before its kernels and copied back after them.
 class ErrorWords
 {
   public:
@@ -341,10 +342,16 @@ class ErrorWords
         auto& words = unused();
         if (words.empty())
         {
+            words.reserve(words.capacity() + 64);
             const BesideCaptures relaxed;
             void* block = nullptr;
-            check_hip(hipHostMalloc(&block, 64 * 64, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
-            words.reserve(words.capacity() + 64);
+            if (hipHostMalloc(&block, 64 * 64, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess)
+            {
+                (void)hipGetLastError(); // not the next launch's error
+                word_.emplace(8, stream);
+                check_hip(hipMemsetAsync(word_->pointer, 0, 8, stream), "hipMemsetAsync");
+                return;
+            }
             for (int i = 0; i < 64; ++i)
             {
                 words.push_back(static_cast<uint32_t*>(block) + 16 * i);
@@ -357,8 +364,11 @@ class ErrorWords
     ~ErrorWords()
     {
         wait();
-        const std::lock_guard<std::mutex> lock(mutex());
-        unused().push_back(host_);
+        if (host_)
+        {
+            const std::lock_guard<std::mutex> lock(mutex());
+            unused().push_back(host_);
+        }
     }
     ErrorWords(const ErrorWords&) = delete;
     ErrorWords& operator=(const ErrorWords&) = delete;
@@ -366,7 +376,14 @@ class ErrorWords
     uint32_t* device() const
     {
         void* p = nullptr;
-        check_hip(hipHostGetDevicePointer(&p, host_, 0), "hipHostGetDevicePointer");
+        if (word_)
+        {
+            p = word_->pointer;
+        }
+        else
+        {
+            check_hip(hipHostGetDevicePointer(&p, host_, 0), "hipHostGetDevicePointer");
+        }
         return static_cast<uint32_t*>(p);
     }
     // Waits for a call that failed on the way: its kernels may still be running.
@@ -380,9 +397,18 @@ class ErrorWords
     // Waits for the call's kernels and fails with `message` if one set its word.
     void check(const char* message)
     {
+        uint32_t word = 0;
+        if (word_)
+        {
+            check_hip(hipMemcpyAsync(&word, word_->pointer, 4, hipMemcpyDeviceToHost, stream_), "read error word");
+        }
         check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
         waited_ = true;
-        require(!*static_cast<volatile uint32_t*>(host_), message);
+        if (!word_)
+        {
+            word = *static_cast<volatile uint32_t*>(host_);
+        }
+        require(!word, message);
     }
 
   private:
@@ -397,6 +423,7 @@ class ErrorWords
         return *words;
     }
     uint32_t* host_ = nullptr;
+    std::optional<AsyncScratch> word_;
     hipStream_t stream_;
     bool waited_ = false;
 };
