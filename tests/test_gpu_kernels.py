@@ -649,7 +649,7 @@ def test_attention_causal_workgroups(torch, native, oracle, heads, hw, lengths, 
         start += length
 
 
-@pytest.mark.parametrize("heads,hw,lengths,sequences", [(8, 64, [256, 250, 193], 480), (8, 64, [384, 330], 236), (8, 64, [200, 70, 64, 1], 800),
+@pytest.mark.parametrize("heads,hw,lengths,sequences", [(8, 64, [256, 250, 193], 480), (8, 64, [384, 330], 536), (8, 64, [200, 70, 64, 1], 800),
                                                         (8, 64, [65, 64, 30], 900), (4, 128, [96, 65, 7], 1200)])
 def test_attention_causal_of_full_devices(torch, native, oracle, heads, hw, lengths, sequences):
     """Launches that fill the device with workgroups of one wave (of 32 queries for the first

@@ -1306,7 +1306,7 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     //   300 x 2             37     29     44     56     34     35    38*
     //   300 x 4             41     49     86     56     35    40*     61
     //   430 x 1             49    27*     37     76     45     39     27
-    //   430 x 20           276    402    653   176*    184    257    390
+    //   430 x 20           276    402    653    176   184*    257    390
     //   862 x 3            162    194    258    153    114   120*    160
     //   2580 x 1           456    473    552    443    319   298*    338
     //   2580 x 3          1294   1414   1650    834   827*    848    979
@@ -1326,22 +1326,20 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     // heads 300 x 2 (1,216 tiles of 8, past the 4 x 8 line at 1,024) would take 29 us on 4 x 8,
     // 120 x 4 and 300 x 4 16 and 35 on 2 x 16.
     //
-    // Launches so large that workgroups of one wave fill the device, however many blocks
-    // the longest chain has, run 64-wide heads on them: no wave holds its slot without a
-    // block or waits for its turn. The largest take 32 queries, whose keys are staged and
-    // widened once for them: a block costs 1.73 times that of 16 there, so that they pay
-    // where the last tiles are nearly full. Lengths are on the device and the rule sees the
-    // longest only, where one long sequence among short ones is its own chain: a block of 32
-    // queries takes 18 us from one wave (16 of 64 queries, before), 10 from two, so one
-    // wave takes 32 only where the number of workgroups alone cost more than that before.
-    // us, 64 queries a workgroup (as it was before the blocks went to waves, and faster
-    // than 2 x 16 here) | 2x16, 1x16, 2x32, 1x32:
-    //   128 x 250       276 |   275   256*   297   260      2580 x 30      8508 |  9482   8814  8030*  7691
-    //   128 x 1000     1070 |  1184  1131   1195  1052*     65 + 64 x 1000  390 |   428   384*   457   382
-    //   176 x 1000     2043 |  2049  1958*  2277  2005      1024 + 12 x 500 375 |   169   222    187   291*
-    //   256 x 1000     3406 |  3981  3840   3698  3328*     1024 + 1 x 30   259 |   130   174    167*  292
-    //   320 x 1000     5009 |  6017  5767   5426  4980*
-    //   1024 x 200     8763 | 10753 10542   9217  8793*
+    // Launches that fill the device many times over run 64-wide heads of up to 5 blocks on
+    // workgroups of one wave: no wave holds its slot without a block or waits for its turn.
+    // The largest take 32 queries, whose keys are staged and widened once for them; a
+    // block costs 1.73 times that of 16 there, so that they pay where the last tiles are
+    // nearly full. Longer histories take two waves then: lengths are on the device and
+    // the rule sees the longest only, and one long sequence among short ones is a chain of
+    // 18 us a block on one wave, 10 on two. us, 64 queries a workgroup (as it was before
+    // the blocks went to waves) | 2x16, 1x16, 2x32, 1x32:
+    //   128 x 250       276 |   275   256*   297   260      1024 x 200     8763 | 10753 10542  9217*  8793
+    //   128 x 1000     1070 |  1184  1131   1195  1052*     2580 x 30      8508 |  9482  8814  8030*  7691
+    //   176 x 1000     2043 |  2049  1958*  2277  2005      512 x 400      4746 |  5743  5527  5027*  4697
+    //   256 x 250       889 |   909   866    931   833*     65 + 64 x 1000  390 |   428   384*  457    382
+    //   256 x 1000     3406 |  3981  3840   3698  3328*     300 + 1 x 500   154 |    77    72   106     91*
+    //   320 x 1000     5009 |  6017  5767   5426  4980*     1024 + 12 x 500 375 |   169   222   187*   291
     // Of 128-wide heads only those of up to 96 rows are faster on one wave (65 + 64 x 1000:
     // 221 | 224, 199*; 96 x 1000 572 | 387, 374*; 128 x 1000 636 | 561*, 575).
     const std::size_t units = std::size_t(compute_units());
@@ -1358,6 +1356,8 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
         const std::size_t columns = (max_length + queries - 1) / queries, each = tile / queries, full = columns / each;
         return each * full * (full + 1) / 2 + columns % each * (full + 1);
     };
+    const std::size_t work = sequences * heads * blocks(32);
+    const bool full = 7 * blocks(32) < 4 * blocks(16); // nearly, the last tile of 32 queries
     const auto tiles = [&](std::size_t queries) { return sequences * heads * ((max_length + queries - 1) / queries); };
     const auto launch = [&](auto rotary, auto plain, int waves, std::size_t queries)
     {
@@ -1389,20 +1389,23 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
         {
             tiles(8) <= 2 * units && max_length > 4 * tile ? variant(eight, eight) : variant(four, eight);
         }
-        else if (tiles(16) >= (5 + 2 * longest) * units && (HW == 64 || max_length <= 96))
+        else if (longest <= 2 ? tiles(16) >= 9 * units && (HW == 64 || max_length <= 96)
+                              : HW == 64 && longest <= 5 && work >= 200 * units)
         {
-            bool wide = false;
             if constexpr (HW == 64)
             {
-                wide = sequences * heads * blocks(32) >= 300 * units && 7 * blocks(32) < 4 * blocks(16);
-                if (wide)
-                {
-                    sequences * heads >= 8 * units ? variant(one, thirty_two) : variant(two, thirty_two);
-                }
+                full && work >= 300 * units ? variant(one, thirty_two) : variant(one, sixteen);
             }
-            if (!wide)
+            else
             {
                 variant(one, sixteen);
+            }
+        }
+        else if (HW == 64 && longest > 5 && full && work >= 700 * units)
+        {
+            if constexpr (HW == 64)
+            {
+                variant(two, thirty_two);
             }
         }
         else if (max_length <= 2 * tile || tiles(16) >= 12 * units ||
