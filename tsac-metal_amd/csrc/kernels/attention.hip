@@ -423,6 +423,7 @@ __global__ __launch_bounds__(decode_waves * 64) void decode_attention_kernel(
 // ------------------------------------------------------------------ prefill
 
 constexpr int tile = 64; // keys of a block
+constexpr unsigned grid_reach = 65535; // query tiles along y; z takes those past it
 
 // 16 bytes at any 2-byte-aligned address.
 __device__ __forceinline__ u32x4 load16(const uint16_t* from)
@@ -521,7 +522,7 @@ template <int HW, int W, int queries, bool Rotary>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) void prefill_kernel(
     const uint16_t* __restrict__ qkv, int width, const int* __restrict__ sequence_start,
     const int* __restrict__ sequence_length, const int* __restrict__ sequence_replay,
-    const uint16_t* __restrict__ rotations, int heads, float scale, uint16_t* __restrict__ out)
+    const uint16_t* __restrict__ rotations, int heads, int columns, float scale, uint16_t* __restrict__ out)
 {
     using Shared = PrefillShared<HW, W, queries>;
     constexpr int per_lane = Shared::per_lane;
@@ -536,9 +537,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 4))) 
     __shared__ Shared shared;
     const int sequence = blockIdx.x / heads, head = blockIdx.x % heads;
     const int length = sequence_length[sequence];
-    // The longest histories first; z takes the tiles past a grid's reach along y.
-    const int q0 = int(gridDim.z * gridDim.y - 1 - (blockIdx.z * gridDim.y + blockIdx.y)) * queries;
-    if (q0 >= length)
+    // The longest histories first.
+    const int q0 = (columns - 1 - int(blockIdx.z * grid_reach + blockIdx.y)) * queries;
+    if (q0 < 0 || q0 >= length)
     {
         return;
     }
@@ -1361,15 +1362,15 @@ void attention_prefill(const uint16_t* qkv, std::size_t width, std::size_t heads
     const auto tiles = [&](std::size_t queries) { return sequences * heads * ((max_length + queries - 1) / queries); };
     const auto launch = [&](auto rotary, auto plain, int waves, std::size_t queries)
     {
-        constexpr std::size_t reach = 65535;
-        const std::size_t columns = (max_length + queries - 1) / queries, layers = (columns + reach - 1) / reach;
+        const std::size_t columns = (max_length + queries - 1) / queries;
         for (std::size_t first = 0; first < sequences; first += slice)
         {
             const dim3 grid(unsigned(std::min(slice, sequences - first) * heads),
-                            unsigned((columns + layers - 1) / layers), unsigned(layers));
+                            unsigned(std::min<std::size_t>(columns, grid_reach)),
+                            unsigned((columns + grid_reach - 1) / grid_reach));
             (rotations ? rotary : plain)<<<grid, 64 * waves, 0, stream>>>(
                 qkv, int(width), sequence_start + first, sequence_length + first, sequence_replay + first, rotations,
-                int(heads), scale, out);
+                int(heads), int(columns), scale, out);
             check_hip(hipGetLastError(), "attention prefill launch");
         }
     };
